@@ -162,6 +162,14 @@ B2G_API int b2g_last_error(b2g_ctx* ctx, char* buf, size_t n);
                           of 224 bytes per contact slot) are allocated when a mask
                           is first set. */
 #define B2G_PARAM_EVENTS 14
+/* B2G_PARAM_GROUP_LOAD   the island solver holds the constraint records of islands
+                          of up to 1022 contacts in registers, in groups of 1 to 8
+                          wavefronts (64 lanes in b2g_island_times), while their
+                          load, in workgroups of 512 lanes weighted by island size,
+                          is at most this (0..2^20, default 768; 0: never, and
+                          never with a heavy class above 9).  Results do not
+                          depend on it. */
+#define B2G_PARAM_GROUP_LOAD 15
 B2G_API int b2g_set_param(b2g_ctx* ctx, int32_t key, int32_t value);
 B2G_API int b2g_get_param(b2g_ctx* ctx, int32_t key, int32_t* value);
 

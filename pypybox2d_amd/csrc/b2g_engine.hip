@@ -92,9 +92,12 @@ constexpr int kProfileBatch = 128;  // steps per event read-back in b2g_profile_
 constexpr int kSizeClasses = 16;
 // q_cls layout: [0, 16) island count per class, [16, 32) cursors,
 // [32] islands in team classes, [33] wavefronts for them,
-// [34, 50) first wavefront per class, [50, 66) first queue entry per class
+// [34, 50) first wavefront per class, [50, 66) first queue entry per class,
+// [66, 82) first workgroup of k_solve_group per class, [82] its workgroups for groups,
+// [83] the lowest class solved by groups (kSizeClasses: k_solve takes every island)
 constexpr int kQHeavy = 2 * kSizeClasses, kQHeavyWaves = kQHeavy + 1, kQWaveBase = kQHeavy + 2,
-              kQBase = kQWaveBase + kSizeClasses, kQcls = kQBase + kSizeClasses;
+              kQBase = kQWaveBase + kSizeClasses, kQGroupBase = kQBase + kSizeClasses,
+              kQGroupBlocks = kQGroupBase + kSizeClasses, kQGroupLow = kQGroupBlocks + 1, kQcls = kQGroupLow + 1;
 
 __host__ __device__ inline int size_class(int nc) {  // floor(log2(nc + 1)), capped
   int c = 0;
@@ -103,6 +106,19 @@ __host__ __device__ inline int size_class(int nc) {  // floor(log2(nc + 1)), cap
 }
 
 constexpr int kSolveBlock = 64;  // k_solve: one wavefront per workgroup
+constexpr int kGroupBlock = 512;      // k_solve_group: eight wavefronts
+constexpr int kGroupWaves = kGroupBlock / 64;
+constexpr int kGroupTopClass = 9;     // the largest islands with a lane per two contacts
+constexpr int kGroupLastClass = 5;     // groups take every island of this class and above, or none
+constexpr int kGroupMaxContacts = (1 << (kGroupTopClass + 1)) - 2;
+
+// Wavefronts of an island of a group class: a lane per contact up to class 8 (510 contacts).
+__host__ __device__ inline int group_waves(int cls) {
+  return cls <= 5 ? 1 : (cls >= 8 ? kGroupWaves : 1 << (cls - 5));
+}
+// Is cls a class whose islands of up to kGroupMaxContacts get two contacts a lane?  The top class
+// holds islands of any size whose state did not fit a team's share (queue_class).
+__host__ __device__ inline bool group_two(int cls) { return cls == kGroupTopClass || cls == kSizeClasses - 1; }
 constexpr int kIslandTimeFields = 6;  // int64 per island of b2g_island_times
 
 // Team size of a heavy size class: 64 lanes from full_cls up, halved per class
@@ -215,6 +231,7 @@ struct Dev {
   int team_full_class;  // ... by a whole wavefront from this class up (half one class below, ...)
   int team_lds;         // LDS bytes per wavefront of teams
   int team_max;         // largest team below the top class (8, 16, 32 or 64)
+  int group_load;       // most load of k_solve_group (plan_groups); 0: none
   // worlds
   const int* w_body_off;
   const int* w_fix_off;
@@ -1782,8 +1799,7 @@ __device__ void init_contact(const Dev<T>& d, const IslandK& c, int bstart, int 
 
 // 5. store_impulses (contact.py:801-806): zip(manifold points, constraint points)
 template <typename T>
-__device__ __forceinline__ void store_impulse(const Dev<T>& d, const IslandK& c, int cstart, int k) {
-  const VC<T>& vc = d.vc[cstart + k];
+__device__ __forceinline__ void store_impulse(const Dev<T>& d, const IslandK& c, int cstart, int k, const VC<T>& vc) {
   const int gs_ = c.cbase + d.i_contacts[cstart + k];
   const int pc = (d.c_state[gs_] >> CS_PC_SHIFT) & 3;
   const int n = pc < vc.npts ? pc : vc.npts;
@@ -1963,7 +1979,7 @@ __device__ void solve_island_joints(const Dev<T>& d, int w, int bstart, int nbi,
     velocity_sweep<T, false>(d, bstart, cstart, nci);
   }
   if (d.i_time) mk.t_vel = (long long)wall_clock64();
-  for (int k = 0; k < nci; ++k) store_impulse(d, c, cstart, k);
+  for (int k = 0; k < nci; ++k) store_impulse(d, c, cstart, k, d.vc[cstart + k]);
   for (int i = 0; i < nbi; ++i) {
     PV<T> p = d.pv[bstart + i];
     integrate_position(p, c.dt);
@@ -2004,7 +2020,7 @@ __device__ void solve_island(const Dev<T>& d, int w, int bstart, int nbi, int cs
   if (c.warm) velocity_sweep<T, true>(d, bstart, cstart, nci);
   for (int it = 0; it < d.vel_iters; ++it) velocity_sweep<T, false>(d, bstart, cstart, nci);
   if (d.i_time) mk.t_vel = (long long)wall_clock64();
-  for (int k = 0; k < nci; ++k) store_impulse(d, c, cstart, k);
+  for (int k = 0; k < nci; ++k) store_impulse(d, c, cstart, k, d.vc[cstart + k]);
   for (int i = 0; i < nbi; ++i) {
     PV<T> p = d.pv[bstart + i];
     integrate_position(p, c.dt);
@@ -2216,7 +2232,7 @@ __device__ void solve_island_team(const Dev<T>& d, int w, int bstart, int nbi, i
   team_sync();
   if (d.i_time) mk.t_vel = (long long)wall_clock64();
   // 5. store impulses, 6. integrate positions (positions to LDS)
-  for (int k = t; k < nci; k += TS) store_impulse(d, c, cstart, k);
+  for (int k = t; k < nci; k += TS) store_impulse(d, c, cstart, k, d.vc[cstart + k]);
   for (int i = t; i < nbi; i += TS) {
     PV<T> p = d.pv[bstart + i];
     p.vx = sx[3 * i];
@@ -2443,7 +2459,9 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
   const int n = *d.q_count;
   const int nh = d.q_cls[kQHeavy];
   const int hw = d.q_cls[kQHeavyWaves];
-  const int nwaves = hw + (n - nh + kSolveBlock - 1) / kSolveBlock;
+  // with groups, only the islands beyond them are left: those of the classes above the groups'
+  const bool grouped = d.q_cls[kQGroupLow] < kSizeClasses;
+  const int nwaves = grouped ? d.q_cls[kQWaveBase + kGroupTopClass] : hw + (n - nh + kSolveBlock - 1) / kSolveBlock;
   const int l = threadIdx.x;
   for (int g = blockIdx.x; g < nwaves; g += gridDim.x) {
     if (g < hw) {
@@ -2464,8 +2482,8 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
         const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
         const bool fits = team_lds_bytes(nbi) <= share;
         SolveMarks mk{0, 0};
-        if (island_has_joints(d, in.x, in.y)) {
-          // k_solve_joints takes it
+        if (island_has_joints(d, in.x, in.y) || (grouped && nci <= kGroupMaxContacts)) {
+          // k_solve_joints or k_solve_group takes it
         } else if (fits) {
           solve_island_team(d, in.x, in.y, nbi, in.w, nci, last_allow, period, team_lds + team * share, t, TS, mk);
           if (d.i_time && t == 0) record_island_time(d, q, t0, nci, nbi, TS, period, mk);
@@ -2477,6 +2495,311 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
       team_sync();
     } else {
       const int q = nh + (g - hw) * kSolveBlock + l;
+      if (q < n) {
+        const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
+        const int4 in = d.qs_isl[q];
+        const int nc = d.qs_nc[q];
+        SolveMarks mk{0, 0};
+        if (!island_has_joints(d, in.x, in.y)) {  // else k_solve_joints takes it
+          solve_island(d, in.x, in.y, in.z & 0xFFFF, in.w, nc & 0x3FFFFFFF, (nc >> 30) & 1, mk);
+          if (d.i_time)
+            record_island_time(d, q, t0, nc & 0x3FFFFFFF, in.z & 0xFFFF, 1, (int)((uint32_t)in.z >> 16), mk);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Island.solve by whole wavefronts, the constraint records held in registers
+//
+// An island gets a group of 1, 2, 4 or 8 wavefronts of a workgroup, enough for a
+// lane per contact (J = 1) or per two contacts (J = 2).  A lane keeps its
+// contact's record, impulses included, in registers over all sweeps, so a
+// solve reads and writes nothing but its two bodies' states in LDS.  The
+// dataflow is the team path's: a contact is ready when its dynamic bodies'
+// counters equal its turn, and at most one pending solve per body can be
+// ready.  Consecutive entries of the level order share a wavefront, so
+// contacts of one level run in one pass.  A body's counter is written after
+// its velocity and read before it; the LDS serves one wavefront's instructions
+// in order, so a lane that sees its turn reads the velocity the turn belongs to.
+// Every lane of a group's wavefronts is resident for the whole solve, the
+// unfinished solve that comes first in the reference's order is always ready,
+// and the polls are capped.  Same arithmetic per contact as the other paths.
+//
+// Bound by the chain of dependent solves (about 9 sweep periods of passes), each some 200 FP64
+// instructions of one wavefront.  A velocity pass takes 0.53 us (FP32 pipeline) or 0.64 us (FP64)
+// where the team path's takes 1.2 us with its records in HBM; the solve stage of one 10-row
+// pyramid 0.86 -> 0.57 ms (FP64), of 67 mixed worlds 3.52 -> 2.78 ms, of 16 small ones
+// 0.38 -> 0.16 ms.  With 128 VGPRs, four wavefronts per SIMD, the record spills and the FP32 pass
+// takes 0.70 us.
+// ---------------------------------------------------------------------------
+struct GroupBody {
+  double x, y, w;
+  int cnt, pad;
+};
+typedef double Dbl2 __attribute__((ext_vector_type(2)));
+static_assert(sizeof(GroupBody) == 32 && offsetof(GroupBody, w) == 16 && offsetof(GroupBody, cnt) == 24, "GroupBody");
+
+// The counters of bodies a and b (LDS addresses), then their states.
+struct GroupRead {
+  int na, nb;
+  Dbl2 pa, pb;
+  double wa, wb;
+};
+__device__ __forceinline__ GroupRead group_read(uint32_t a, uint32_t b) {
+  GroupRead r;
+  asm volatile(
+      "ds_read_b32 %0, %6 offset:24\n\t"
+      "ds_read_b32 %1, %7 offset:24\n\t"
+      "ds_read_b128 %2, %6\n\t"
+      "ds_read_b64 %3, %6 offset:16\n\t"
+      "ds_read_b128 %4, %7\n\t"
+      "ds_read_b64 %5, %7 offset:16\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r.na), "=&v"(r.nb), "=&v"(r.pa), "=&v"(r.wa), "=&v"(r.pb), "=&v"(r.wb)
+      : "v"(a), "v"(b)
+      : "memory");
+  return r;
+}
+__device__ __forceinline__ void group_write(uint32_t a, double x, double y, double w, int cnt) {
+  const Dbl2 p = {x, y};
+  asm volatile(
+      "ds_write_b128 %0, %1\n\t"
+      "ds_write_b64 %0, %2 offset:16\n\t"
+      "ds_write_b32 %0, %3 offset:24"
+      :
+      : "v"(a), "v"(p), "v"(w), "v"(cnt)
+      : "memory");
+}
+
+// The wavefronts of one group meet: *bar counts arrivals, `due` the arrivals a wavefront waits for.
+__device__ __forceinline__ void group_sync(int* bar, int& due, int waves) {
+  team_sync();
+  if (waves == 1) return;
+  due += waves;
+  if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(bar, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  while (__hip_atomic_load(bar, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < due) __builtin_amdgcn_s_sleep(1);
+  team_sync();
+}
+
+constexpr int kGroupPolls = 1 << 22;  // polls without an end of the sweeps: WERR_SCHEDULE
+
+template <typename T, int J>
+__device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int bstart, int nbi, int cstart, int nci,
+                                                   int last_allow, GroupBody* st, int* bar, double* red, int t,
+                                                   int waves, SolveMarks& mk) {
+  const IslandK c = island_k(d, w, bstart);
+  const int TS = waves * 64, lane = t & 63, wv = t >> 6;
+  int due = 0;
+  // slot nbi: a static side's state, zero and always at turn 0; slot nbi + 1 takes its writes
+  for (int i = t; i < nbi + 2; i += TS) {
+    double vx = 0.0, vy = 0.0, vw = 0.0;
+    if (i < nbi) {
+      const PV<T> p = d.pv[bstart + i];
+      vx = p.vx;
+      vy = p.vy;
+      vw = p.w;
+    }
+    st[i].x = vx;
+    st[i].y = vy;
+    st[i].w = vw;
+    st[i].cnt = 0;
+  }
+  const uint32_t* order = d.i_order + cstart;
+  const uint32_t base = lds_addr(st), zero = base + 32u * nbi, trash = zero + 32u;
+  int ks[J];
+  bool has[J];
+  uint32_t ra_[J], rb_[J], wa_[J], wb_[J];  // LDS addresses: the bodies' states, where to write them
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int p = wv * 64 * J + j * 64 + lane;
+    has[j] = p < nci;
+    ks[j] = has[j] ? (int)(order[p] & 0xFFFFu) : 0;
+  }
+  // 3 + 4. warm start and velocity sweeps
+  const int nsw = d.vel_iters + (c.warm ? 1 : 0);
+  {
+    VC<T> cur[J];
+    int ta[J], tb[J], left[J];
+    bool pend = false;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      cur[j] = d.vc[cstart + ks[j]];
+      const int ia = cur[j].ia, ib = cur[j].ib;
+      ra_[j] = ia >= 0 ? base + 32u * ia : zero;
+      rb_[j] = ib >= 0 ? base + 32u * ib : zero;
+      wa_[j] = ia >= 0 ? ra_[j] : trash;
+      wb_[j] = ib >= 0 ? rb_[j] : trash;
+      ta[j] = cur[j].rka & 0xFFFF;
+      tb[j] = cur[j].rkb & 0xFFFF;
+      left[j] = has[j] ? nsw : 0;
+      pend |= left[j] > 0;
+    }
+    group_sync(bar, due, waves);
+    int poll = 0;
+    while (wave_any(pend) && poll < kGroupPolls) {
+      ++poll;
+      pend = false;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const GroupRead r = group_read(ra_[j], rb_[j]);
+        if ((left[j] > 0) & (r.na == ta[j]) & (r.nb == tb[j])) {
+          V2d va = v2<double>(r.pa.x, r.pa.y), vb = v2<double>(r.pb.x, r.pb.y);
+          double wa = r.wa, wb = r.wb;
+          if (c.warm && left[j] == nsw) warm_contact(cur[j], va, wa, vb, wb);
+          else solve_contact_velocity(cur[j], va, wa, vb, wb);
+          group_write(wa_[j], va.x, va.y, wa, ta[j] + 1);
+          group_write(wb_[j], vb.x, vb.y, wb, tb[j] + 1);
+          ta[j] += (int)((unsigned)cur[j].rka >> 16);
+          tb[j] += (int)((unsigned)cur[j].rkb >> 16);
+          --left[j];
+        }
+        pend |= left[j] > 0;
+      }
+    }
+    if (pend) atomicOr(&d.w_err[w], WERR_SCHEDULE);  // poll limit reached
+    if (d.i_time) mk.t_vel = (long long)wall_clock64();
+    // 5. store impulses
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      if (has[j]) store_impulse(d, c, cstart, ks[j], cur[j]);
+  }
+  group_sync(bar, due, waves);
+  // 6. integrate positions (positions to LDS)
+  for (int i = t; i < nbi; i += TS) {
+    PV<T> p = d.pv[bstart + i];
+    p.vx = st[i].x;
+    p.vy = st[i].y;
+    p.w = st[i].w;
+    integrate_position(p, c.dt);
+    d.pv[bstart + i] = p;
+    st[i].x = p.cx;
+    st[i].y = p.cy;
+    st[i].w = p.a;
+    st[i].cnt = 0;
+  }
+  // 7. position iterations with early exit, one dataflow sweep each
+  bool position_solved = false;
+  {
+    PC<T> cur[J];
+    int ta[J], tb[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      cur[j] = d.pc[cstart + ks[j]];
+      ta[j] = cur[j].rka & 0xFFFF;
+      tb[j] = cur[j].rkb & 0xFFFF;
+    }
+    group_sync(bar, due, waves);
+    for (int it = 0; it < d.pos_iters && !position_solved; ++it) {  // group-uniform
+      if (d.i_time) mk.npos = it + 1;
+      T min_sep = 0;
+      bool todo[J], pend = false;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        todo[j] = has[j];
+        pend |= has[j];
+      }
+      int poll = 0;
+      while (wave_any(pend) && poll < kGroupPolls) {
+        ++poll;
+        pend = false;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const GroupRead r = group_read(ra_[j], rb_[j]);
+          if (todo[j] & (r.na == ta[j]) & (r.nb == tb[j])) {
+            const bool sa = cur[j].ia < 0, sb = cur[j].ib < 0;
+            double ax = sa ? cur[j].scx : r.pa.x, ay = sa ? cur[j].scy : r.pa.y, aa = sa ? cur[j].sa : r.wa;
+            double bx = sb ? cur[j].scx : r.pb.x, by = sb ? cur[j].scy : r.pb.y, ab = sb ? cur[j].sa : r.wb;
+            solve_contact_position(cur[j], ax, ay, aa, bx, by, ab, min_sep);
+            group_write(wa_[j], ax, ay, aa, ta[j] + 1);
+            group_write(wb_[j], bx, by, ab, tb[j] + 1);
+            ta[j] += (int)((unsigned)cur[j].rka >> 16);
+            tb[j] += (int)((unsigned)cur[j].rkb >> 16);
+            todo[j] = false;
+          }
+          pend |= todo[j];
+        }
+      }
+      if (pend) atomicOr(&d.w_err[w], WERR_SCHEDULE);
+      min_sep = team_min(min_sep, 64);  // the sequential loop's min_separation
+      double* slot = red + (it & 1) * kGroupWaves;
+      if (lane == 0) slot[wv] = (double)min_sep;
+      group_sync(bar, due, waves);
+      for (int k = 0; k < waves; ++k) min_sep = pmin(min_sep, (T)slot[k]);
+      if (min_sep >= -(T)(3.0 * LINEAR_SLOP)) position_solved = true;
+    }
+  }
+  // 8. copy back (a group's last sweep has ended: its wavefronts met after it)
+  group_sync(bar, due, waves);
+  for (int i = t; i < nbi; i += TS) {
+    PV<T> p = d.pv[bstart + i];
+    p.cx = st[i].x;
+    p.cy = st[i].y;
+    p.a = st[i].w;
+    write_back(d, c, bstart, i, p);
+  }
+  // 9. sleep (each lane reads back only the bodies it wrote)
+  if (c.wflags & WF_ALLOW_SLEEP) {
+    double min_sleep = 1.0e300;
+    for (int i = t; i < nbi; i += TS) min_sleep = pmin(min_sleep, sleep_body(d, c, bstart, i, last_allow));
+    min_sleep = team_min(min_sleep, 64);
+    double* slot = red + 2 * kGroupWaves;
+    if (lane == 0) slot[wv] = min_sleep;
+    group_sync(bar, due, waves);
+    for (int k = 0; k < waves; ++k) min_sleep = pmin(min_sleep, slot[k]);
+    if (min_sleep >= TIME_TO_SLEEP && position_solved && nbi > 0 && t == (nbi - 1) % TS)
+      sleep_last(d, c, bstart, nbi);
+  }
+}
+
+// One workgroup of k_solve_group: its islands of class cls, 8 / group_waves(cls) at a time.
+template <typename T, int J>
+__device__ __forceinline__ void solve_group_block(const Dev<T>& d, int cls, int g, GroupBody* st, int* bar,
+                                                  double (*red)[3 * kGroupWaves]) {
+  const int waves = J == 2 ? kGroupWaves : group_waves(cls), per = kGroupWaves / waves;
+  const int team = (threadIdx.x >> 6) / waves, t = threadIdx.x - team * waves * 64;
+  const int q = d.q_cls[kQBase + cls] + (g - d.q_cls[kQGroupBase + cls]) * per + team;
+  if (q >= d.q_cls[kQBase + cls] + d.q_cls[cls]) return;
+  const int4 in = d.qs_isl[q];
+  const int nc = d.qs_nc[q];
+  const int nbi = in.z & 0xFFFF, nci = nc & 0x3FFFFFFF, last_allow = (nc >> 30) & 1;
+  // islands with joints are left to k_solve_joints, larger ones of the top class to k_solve
+  if (nci > kGroupMaxContacts || island_has_joints(d, in.x, in.y)) return;
+  const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
+  SolveMarks mk{0, 0};
+  solve_island_group<T, J>(d, in.x, in.y, nbi, in.w, nci, last_allow, st + team * (waves * 64 * J + 1), &bar[team],
+                           red[team], t, waves, mk);
+  if (d.i_time && t == 0)
+    record_island_time(d, q, t0, nci, nbi, kSolveBlock, (int)((uint32_t)in.z >> 16), mk);
+}
+
+// Where plan_groups has chosen groups: the group classes from the largest islands down, then the
+// smaller islands one lane each.
+template <typename T>
+__global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_eu(2))) k_solve_group(Dev<T> d) {
+  // a group of W wavefronts has at most 64 W J - 1 bodies (they hang together by 64 W J - 2
+  // contacts or fewer), and two slots more
+  __shared__ __align__(16) GroupBody st[2 * kGroupBlock + kGroupWaves];
+  __shared__ double red[kGroupWaves][3 * kGroupWaves];
+  __shared__ int bar[kGroupWaves];
+  const int low = d.q_cls[kQGroupLow];
+  if (low >= kSizeClasses) return;  // k_solve takes every island
+  const int groups = d.q_cls[kQGroupBlocks];
+  const int n = *d.q_count, light = d.q_cls[kQBase + low] + d.q_cls[low];
+  const int blocks = groups + (n - light + kGroupBlock - 1) / kGroupBlock;
+  for (int g = blockIdx.x; g < blocks; g += gridDim.x) {
+    if (g < groups) {
+      int cls = low;  // the classes own consecutive workgroup ranges, highest class first
+      while (cls < kGroupTopClass && g < d.q_cls[kQGroupBase + cls]) ++cls;
+      if (g < d.q_cls[kQGroupBase + cls]) cls = kSizeClasses - 1;
+      if (threadIdx.x < kGroupWaves) bar[threadIdx.x] = 0;
+      __syncthreads();
+      if (group_two(cls)) solve_group_block<T, 2>(d, cls, g, st, bar, red);
+      else solve_group_block<T, 1>(d, cls, g, st, bar, red);
+      __syncthreads();  // the next islands reuse the LDS
+    } else {
+      const int q = light + (g - groups) * kGroupBlock + (int)threadIdx.x;
       if (q < n) {
         const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
         const int4 in = d.qs_isl[q];
@@ -4608,6 +4931,33 @@ __global__ void k_disable(Dev<T> d, const int* ws, int n) {
   if (st & CS_LIVE) d.c_state[s] = st & ~CS_ENABLED;
 }
 
+// Which islands k_solve_group takes.  Its workgroups fill a compute unit's registers, so an island
+// waits for one where the team path's wavefronts would already run: groups pay while the chip is
+// not full of them.  Their load is the workgroups weighted by the length of their islands (measured
+// means 1.0 ms for class 8, 0.4, 0.22 and 0.12 ms for 7, 6 and 5, 1.9 ms for 9), in eighths of a
+// workgroup of class 8.  Solve stage in ms with and without groups, mixed worlds of 32 to 512 bodies:
+// 256 worlds 2.60 / 3.26, 509 2.58 / 3.34, 700 (load about 630) 3.03 / 3.55, 1000 (about 900)
+// 4.07 / 3.65; 3001 long-tailed worlds (about 520) 2.90 / 3.41.  Every class from 5 up has to fit
+// (k_solve has teams for them); smaller islands get a wavefront each while there is room, else a lane.
+template <typename T>
+__device__ void plan_groups(const Dev<T>& d) {
+  int blocks = 0, load = 0, low = kSizeClasses;
+  if (d.group_load > 0 && d.heavy_class <= kGroupTopClass) {
+    for (int c = kSizeClasses - 1; c > 0; c = c == kSizeClasses - 1 ? kGroupTopClass : c - 1) {
+      const int n = d.q_cls[c];
+      const int need = group_two(c) ? n : (n * group_waves(c) + kGroupWaves - 1) / kGroupWaves;
+      load += need * (group_two(c) ? 16 : (c > 5 ? 1 << (c - 5) : 1));
+      if (load > 8 * d.group_load) break;
+      d.q_cls[kQGroupBase + c] = blocks;
+      blocks += need;
+      low = c;
+    }
+    if (low > kGroupLastClass) low = kSizeClasses;
+  }
+  d.q_cls[kQGroupBlocks] = blocks;
+  d.q_cls[kQGroupLow] = low;
+}
+
 // Orders the island queue by size class, largest first, so that the lanes of
 // a wave of k_solve carry islands of similar length.  Each block takes a
 // contiguous chunk of the queue, counts its classes in LDS and reserves its
@@ -4633,6 +4983,7 @@ __global__ void k_order_islands(Dev<T> d) {
         d.q_cls[kQHeavyWaves] = waves;
       }
     }
+    if (blockIdx.x == 0) plan_groups(d);
   }
   __syncthreads();
   const int n = *d.q_count;
@@ -4670,10 +5021,10 @@ template <typename T>
 __global__ void __launch_bounds__(kPrefixBlock) k_order_team_islands(Dev<T> d) {
   __shared__ int bins[kTeamSortBins], scan[kPrefixBlock];
   const int c = blockIdx.x;
-  if (c < d.heavy_class) return;
+  if (c < d.heavy_class && c < d.q_cls[kQGroupLow]) return;
   const int b = d.q_cls[kQBase + c], n = d.q_cls[c];
   if (n < 2) return;
-  const int TS = team_size(c, d.team_full_class, d.team_max);
+  const int TS = c >= d.q_cls[kQGroupLow] ? 2 * kGroupBlock : team_size(c, d.team_full_class, d.team_max);
   auto bin_of = [&](const int4& in, int nc) {
     const int est = team_island_length(in, nc, TS);
     return kTeamSortBins - 1 - (est < kTeamSortBins - 1 ? est : kTeamSortBins - 1);
@@ -4917,6 +5268,7 @@ struct b2g_ctx {
   int team_full_class = 9;
   int team_lds = 24576;
   int team_max = 32;
+  int group_load = 768;                  // B2G_PARAM_GROUP_LOAD
   int pairs_wide = kPairsWideMaxPerCu;   // B2G_PARAM_PAIRS_WIDE
   int islands_wide = kIslandsWidePerCu;  // B2G_PARAM_ISLANDS_WIDE
   int collide_block = kBlock;            // B2G_PARAM_COLLIDE_BLOCK
@@ -5635,6 +5987,7 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
   d.vel_iters = vi;
   d.pos_iters = pi;
   d.heavy_class = ctx->heavy_class;
+  d.group_load = ctx->group_load;
   d.team_full_class = ctx->team_full_class;
   d.team_lds = ctx->team_lds;
   d.team_max = ctx->team_max;
@@ -5732,7 +6085,21 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
     hipLaunchKernelGGL(k_prep_bodies<T>, dim3((unsigned)pgrid), dim3(kBlock), 0, st, d);
     hipLaunchKernelGGL(k_prep_contacts<T>, dim3((unsigned)kPrepGrid), dim3(kBlock), 0, st, d);
     const int swaves = std::max(1, std::min((ctx->nb + kSolveBlock - 1) / kSolveBlock, ctx->solve_grid));
-    hipLaunchKernelGGL(k_solve<T>, dim3(swaves), dim3(kSolveBlock), ctx->team_lds, st, d);
+    // k_solve has work beside the groups' only in worlds that can hold an island too large for them
+    const bool beside = ctx->group_load > 0 && ctx->max_ccap > kGroupMaxContacts;
+    if (beside) {
+      HIPCHK(hipEventRecord(ctx->fork_ev, st));
+      HIPCHK(hipStreamWaitEvent(ctx->aux[0], ctx->fork_ev, 0));
+    }
+    hipLaunchKernelGGL(k_solve<T>, dim3(swaves), dim3(kSolveBlock), ctx->team_lds, beside ? ctx->aux[0] : st, d);
+    if (ctx->group_load > 0) {
+      const int ggrid = std::max(1, std::min(ctx->nb, 4096));
+      hipLaunchKernelGGL(k_solve_group<T>, dim3(ggrid), dim3(kGroupBlock), 0, st, d);
+    }
+    if (beside) {
+      HIPCHK(hipEventRecord(ctx->join_ev[0], ctx->aux[0]));
+      HIPCHK(hipStreamWaitEvent(st, ctx->join_ev[0], 0));
+    }
     if (ctx->nj > 0)
       hipLaunchKernelGGL(k_solve_joints<T>, dim3((unsigned)std::max(1, (ctx->nb + 63) / 64)), dim3(64), 0, st, d);
     if (part == PART_ISLANDS) {
@@ -6346,6 +6713,7 @@ B2G_API int b2g_set_param(b2g_ctx* ctx, int32_t key, int32_t value) {
     case B2G_PARAM_SOLVE_GRID: slot = &ctx->solve_grid; lo = 1; hi = 1 << 30; break;
     case B2G_PARAM_ISLAND_TIMES: slot = &ctx->island_times; lo = 0; hi = 1; break;
     case B2G_PARAM_TEAM_MAX: slot = &ctx->team_max; lo = 8; hi = kSolveBlock; break;
+    case B2G_PARAM_GROUP_LOAD: slot = &ctx->group_load; lo = 0; hi = 1 << 20; break;
     case B2G_PARAM_PAIRS_WIDE: slot = &ctx->pairs_wide; lo = 0; hi = 32; break;
     case B2G_PARAM_ISLANDS_WIDE: slot = &ctx->islands_wide; lo = 0; hi = 32; break;
     case B2G_PARAM_COLLIDE_BLOCK: slot = &ctx->collide_block; lo = 64; hi = 512; break;
@@ -6392,6 +6760,7 @@ B2G_API int b2g_get_param(b2g_ctx* ctx, int32_t key, int32_t* value) {
     case B2G_PARAM_SOLVE_GRID: *value = ctx->solve_grid; return B2G_OK;
     case B2G_PARAM_ISLAND_TIMES: *value = ctx->island_times; return B2G_OK;
     case B2G_PARAM_TEAM_MAX: *value = ctx->team_max; return B2G_OK;
+    case B2G_PARAM_GROUP_LOAD: *value = ctx->group_load; return B2G_OK;
     case B2G_PARAM_PAIRS_WIDE: *value = ctx->pairs_wide; return B2G_OK;
     case B2G_PARAM_ISLANDS_WIDE: *value = ctx->islands_wide; return B2G_OK;
     case B2G_PARAM_COLLIDE_BLOCK: *value = ctx->collide_block; return B2G_OK;

@@ -1,0 +1,68 @@
+"""The register-resident island solve (groups of wavefronts, B2G_PARAM_GROUP_LOAD) against the
+team and lane paths: the same solves in the same order, so the same bits, at the edges of its
+classes (62 / 63, 126 / 127, 254 / 255, 510 / 511 and 1022 / 1023 contacts an island)."""
+import numpy as np
+import pytest
+
+from pypybox2d_amd import _native as N
+from pypybox2d_amd import builder, layout as L, scenes
+
+pytestmark = pytest.mark.gpu
+DT = 1.0 / 60
+
+PATHS = {"groups": {"group_load": 1 << 20}, "default": {}, "few": {"group_load": 3},
+         "teams64": {"group_load": 0, "heavy_class": 0, "team_full_class": 0},
+         "teams8": {"group_load": 0, "heavy_class": 0, "team_full_class": 16},
+         "fallback": {"group_load": 0, "heavy_class": 3, "team_lds": 4096},
+         "pairs": {"group_load": 0, "heavy_class": 5, "team_full_class": 9, "team_max": 32},
+         "lanes": {"heavy_class": 16}}
+
+
+def _run(prec, state, vel_iters=8, pos_iters=3):
+    out, times = {}, {}
+    for name, params in PATHS.items():
+        e = N.Engine(prec)
+        for k, v in params.items():
+            e.set_param(k, v)
+        e.set_param("island_times", 1)
+        e.upload(state)
+        for _ in range(2):
+            e.step(DT, vel_iters, pos_iters)
+        e.step_n(2, DT, vel_iters, pos_iters, graph=True)
+        out[name], times[name] = e.download(), e.island_times()
+        print(prec, name, "done", flush=True)
+        e.close()
+    ref = out["lanes"]
+    for name, st in out.items():
+        for f in ("body_d", "body_i", "fix_d", "con_d", "con_i"):
+            assert np.array_equal(getattr(st, f), getattr(ref, f)), (name, f)
+    return times
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_islands_around_the_class_limits(prec):
+    """Pyramids of 2 to 34 rows: islands of 3 to over 1022 contacts, one- and two-point manifolds."""
+    rows = (2, 3, 5, 7, 8, 9, 11, 12, 13, 15, 18, 19, 22, 26, 31, 34)
+    e = N.Engine(prec)
+    e.upload(builder.scenes_batch([dict(scenes.pyramid(n), do_sleep=n % 2 == 0) for n in rows]))
+    e.step_n(40, DT, 8, 3, graph=True)
+    state = e.download()
+    e.close()
+    times = _run(prec, state)
+    n = times["groups"][:, 2]
+    assert n.max() > 1022 and set(times["groups"][n <= 1022, 4].tolist()) <= {1, 64}
+    assert np.all(times["groups"][(n >= 31) & (n <= 1022), 4] == 64)
+
+
+@pytest.mark.parametrize("prec,iters", [("fp64", (8, 3)), ("fp32", (8, 3)), ("fp32", (1, 0)), ("fp64", (0, 1))])
+def test_piles_static_sides_and_iteration_counts(prec, iters):
+    """Mixed piles (circles, polygons and edges on static ground), with and without warm starting."""
+    counts = [16, 40, 96, 180, 260, 420, 512]
+    batch = builder.scenes_batch([scenes.batch_world(9, w, n) for w, n in enumerate(counts)])
+    e = N.Engine(prec)
+    e.upload(batch)
+    e.step_n(150, DT, 8, 3, graph=True)
+    state = e.download()
+    e.close()
+    state.world_i[::2, L.WI_FLAGS] &= ~L.WF_WARM_STARTING
+    _run(prec, state, *iters)
