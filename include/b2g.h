@@ -91,6 +91,10 @@ B2G_API int b2g_counts(b2g_ctx* ctx, int32_t* counts);
    Replaces reading Body/Contact/Manifold/Joint attributes after World.step. */
 B2G_API int b2g_download(b2g_ctx* ctx, b2g_batch_out* out);
 
+/* memcpy of host arrays by up to 8 threads (from 4 MB on), for the copies of a
+   state that a caller keeps beside the downloaded one. */
+B2G_API int b2g_host_copy(void* dst, const void* src, size_t bytes);
+
 B2G_API int b2g_last_error(b2g_ctx* ctx, char* buf, size_t n);
 
 /* Launch shape of the island solver.  The reference solves islands one after

@@ -24,7 +24,7 @@ EXPORTS = ("b2g_version", "b2g_create", "b2g_destroy", "b2g_upload", "b2g_step",
            "b2g_counts", "b2g_download", "b2g_last_error", "b2g_set_param", "b2g_get_param", "b2g_profile_step",
            "b2g_island_times", "b2g_narrowphase", "b2g_pairs", "b2g_stats", "b2g_query_aabb", "b2g_ray_cast",
            "b2g_pairs_noalloc", "b2g_events", "b2g_pair_search", "b2g_new_contacts", "b2g_drop_contacts",
-           "b2g_step_collide", "b2g_step_solve", "b2g_disable_contacts", "b2g_solve_islands")
+           "b2g_step_collide", "b2g_step_solve", "b2g_disable_contacts", "b2g_solve_islands", "b2g_host_copy")
 
 # keys of b2g_set_param / b2g_get_param: the solver's launch shape, island timing, and the
 # resident solver wavefronts per compute unit and the search launches per step (both read only)
@@ -91,10 +91,23 @@ def load(path: Optional[str] = None):
     lib.b2g_step_collide.argtypes = [vp, f64, ctypes.c_int, ctypes.c_int]
     lib.b2g_step_solve.argtypes = [vp]
     lib.b2g_disable_contacts.argtypes = [vp, ctypes.c_int32, vp, vp]
+    lib.b2g_host_copy.argtypes = [vp, vp, ctypes.c_size_t]
     lib.b2g_solve_islands.argtypes = [vp, f64, ctypes.c_int, ctypes.c_int]
     _ = i32
     _lib = lib
     return lib
+
+
+COPY_THREADED = 4 << 20  # bytes from which a copy is worth threads
+
+
+def host_copy(src: np.ndarray, out: np.ndarray) -> np.ndarray:
+    """Copies src into out (of its shape), large arrays by several threads."""
+    if src.nbytes < COPY_THREADED or src.dtype != out.dtype or not (src.flags.c_contiguous and out.flags.c_contiguous):
+        np.copyto(out, src)
+    else:
+        load().b2g_host_copy(out.ctypes.data, src.ctypes.data, src.nbytes)
+    return out
 
 
 class Engine:
@@ -112,6 +125,7 @@ class Engine:
             raise B2GError(rc, "b2g_create")
         self.h = h
         self._like: Optional[L.BatchArrays] = None
+        self._pool = L.ArrayPool()
 
     def _check(self, rc: int, what: str) -> None:
         if rc:
@@ -154,7 +168,8 @@ class Engine:
 
     def download(self) -> L.BatchArrays:
         c = self.counts()
-        out = L.OutBuffers(self._like, con_cap=int(c[2]) + 16, move_cap=int(c[1]) + 16)
+        out = L.OutBuffers(self._like, con_cap=int(c[2]) + 16, move_cap=int(c[1]) + 16,
+                           empty=self._pool.get, copy=host_copy)
         self._check(self.lib.b2g_download(self.h, ctypes.byref(out.struct)), "download")
         return out.to_batch()
 

@@ -9,8 +9,9 @@ per-world offset arrays; ``BatchArrays.as_struct`` exposes them as the
 from __future__ import annotations
 
 import ctypes
+import sys
 from dataclasses import dataclass, field
-from typing import List, Optional
+from typing import Dict, List, Optional
 
 import numpy as np
 
@@ -278,10 +279,36 @@ def concat(worlds: List[BatchArrays]) -> BatchArrays:
                        np.concatenate([w.joint_i for w in worlds]).reshape(-1, JOINT_NI).astype(np.int32))
 
 
+class ArrayPool:
+    """Memory of large arrays, used again once nothing refers to it: fresh pages cost more to touch
+    than a readout takes to write (4 GB/s on one thread).  At most two blocks per name are kept, so
+    that the next array can be filled while the last one is still held."""
+    SMALL = 1 << 16  # bytes below which the allocator does as well
+
+    def __init__(self):
+        self._blocks: Dict[str, List[np.ndarray]] = {}
+
+    def get(self, name: str, shape, dtype) -> np.ndarray:
+        """An array with arbitrary contents."""
+        n = int(np.prod(shape))
+        if n * np.dtype(dtype).itemsize < self.SMALL:
+            return np.empty(shape, dtype)
+        blocks = self._blocks.setdefault(name, [])
+        for k in range(len(blocks)):
+            # referred to by this list alone: no array made of it is left
+            if sys.getrefcount(blocks[k]) == 2 and n <= blocks[k].size <= 2 * n and blocks[k].dtype == dtype:
+                return blocks[k][:n].reshape(shape)
+        block = np.empty(n + n // 16, dtype)
+        blocks.append(block)
+        del blocks[:-2]
+        return block[:n].reshape(shape)
+
+
 class OutBuffers:
     """Writable output arrays for a batch (``b2g_batch_out``)."""
 
-    def __init__(self, like: BatchArrays, con_cap: Optional[int] = None, move_cap: Optional[int] = None):
+    def __init__(self, like: BatchArrays, con_cap: Optional[int] = None, move_cap: Optional[int] = None,
+                 empty=lambda name, shape, dtype: np.zeros(shape, dtype), copy=lambda src, out: np.copyto(out, src)):
         nw = like.n_worlds
         nb = like.body_d.shape[0]
         nf = like.fix_d.shape[0]
@@ -291,13 +318,15 @@ class OutBuffers:
         self.move_off = np.zeros(nw + 1, np.int32)
         self.world_d = like.world_d.copy()
         self.world_i = like.world_i.copy()
-        self.body_d = np.zeros((nb, BODY_ND))
-        self.body_i = np.zeros((nb, BODY_NI), np.int32)
-        self.fix_d = like.fix_d.copy()
-        self.fix_i = like.fix_i.copy()
-        self.con_d = np.zeros((self.con_cap, CON_ND))
-        self.con_i = np.zeros((self.con_cap, CON_NI), np.int32)
-        self.move = np.zeros(self.move_cap, np.int32)
+        self.body_d = empty("body_d", (nb, BODY_ND), np.float64)
+        self.body_i = empty("body_i", (nb, BODY_NI), np.int32)
+        self.fix_d = empty("fix_d", like.fix_d.shape, np.float64)
+        self.fix_i = empty("fix_i", like.fix_i.shape, np.int32)
+        copy(like.fix_d, self.fix_d)
+        copy(like.fix_i, self.fix_i)
+        self.con_d = empty("con_d", (self.con_cap, CON_ND), np.float64)
+        self.con_i = empty("con_i", (self.con_cap, CON_NI), np.int32)
+        self.move = empty("move", (self.move_cap,), np.int32)
         self.body_off = like.body_off.copy()
         self.fix_off = like.fix_off.copy()
         self.joint_off = np.ascontiguousarray(like.joint_off, dtype=np.int32).copy()
@@ -309,10 +338,10 @@ class OutBuffers:
                                 _ptr(self.move), _ptr(self.joint_d), _ptr(self.joint_i))
 
     def to_batch(self) -> BatchArrays:
+        """The batch read, in these arrays (not copies of them)."""
         nc = int(self.con_off[-1])
         nm = int(self.move_off[-1])
-        return BatchArrays(self.body_off.copy(), self.fix_off.copy(), self.con_off.copy(),
-                           self.move_off.copy(), self.world_d.copy(), self.world_i.copy(),
-                           self.body_d.copy(), self.body_i.copy(), self.fix_d.copy(), self.fix_i.copy(),
-                           self.con_d[:nc].copy(), self.con_i[:nc].copy(), self.move[:nm].copy(),
-                           self.joint_off.copy(), self.joint_d.copy(), self.joint_i.copy())
+        return BatchArrays(self.body_off, self.fix_off, self.con_off, self.move_off, self.world_d, self.world_i,
+                           self.body_d, self.body_i, self.fix_d, self.fix_i,
+                           self.con_d[:nc], self.con_i[:nc], self.move[:nm],
+                           self.joint_off, self.joint_d, self.joint_i)

@@ -24,7 +24,7 @@ from __future__ import annotations
 from typing import Dict, List, Optional
 
 from . import layout as L
-from ._native import B2G_E_CAPACITY, B2GError, Engine
+from ._native import B2G_E_CAPACITY, B2GError, Engine, host_copy
 
 MAX_REGROW = 6
 MAX_LOG = 256  # operations kept for a replay before the state is checkpointed by a download
@@ -40,6 +40,7 @@ class Stepper(object):
                                      contact_extra=self.contact_extra)
         self.params: Dict[str, int] = {}
         self._ckpt: Optional[L.BatchArrays] = None
+        self._pool = L.ArrayPool()  # memory of _ckpt's arrays that change size
         self._log: List[tuple] = []  # operations since _ckpt: ("step", n, dt, vi, pi), ("pairs",), ("drop", w, j)
         self.regrows = 0
         self.on_regrow = None  # called with the new Engine after a regrow
@@ -58,9 +59,30 @@ class Stepper(object):
     def download(self) -> L.BatchArrays:
         st = self.engine.download()
         if not self._split:  # a state between a step's two parts is no replay start
-            self._ckpt = st.copy()
+            self._keep(st)
             self._log = []
         return st
+
+    def _keep(self, st: L.BatchArrays) -> None:
+        """Makes the downloaded st the replay start: its arrays are copied over the last start's where
+        they fit (the caller may change st).  A fixture's record changes in its fat AABB alone."""
+        old = self._ckpt
+        if old is None or old.fix_d.shape != st.fix_d.shape:
+            self._ckpt = st.copy()
+            return
+        new = {}
+        for n in L.ALL_FIELDS:
+            src, out = getattr(st, n), getattr(old, n)
+            if n == "fix_d":
+                continue
+            if out.shape != src.shape:  # the contacts and moves of another frame
+                setattr(old, n, None)
+                out = None
+                out = self._pool.get(n, src.shape, src.dtype)
+            new[n] = host_copy(src, out)
+        fat = slice(L.FD_FAT_LX, L.FD_FAT_LX + 4)
+        old.fix_d[:, fat] = st.fix_d[:, fat]
+        self._ckpt = L.BatchArrays(fix_d=old.fix_d, **new)
 
     def record(self, n: int, dt: float, vel_iters: int, pos_iters: int) -> None:
         """Logs n steps that were launched on the engine directly (e.g. by the launch tuner)."""
