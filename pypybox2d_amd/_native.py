@@ -236,7 +236,7 @@ class Engine:
                 continue
             self._check(rc, "ray_cast")
             m = int(n[0])
-            return oi[:m].copy(), od[:m].copy()
+            return (oi, od) if m == cap else (oi[:m].copy(), od[:m].copy())
 
     def events(self):
         """The contact listener's records of the last step (b2g_events; kinds enabled with

@@ -37,7 +37,7 @@ def test_every_world_reads_as_it_does_alone(prec, copies):
 
 
 def test_dropped_contacts_are_left_out_in_place():
-    batch = builder.scenes_batch([scenes.batch_world(5, k, 40 + k) for k in range(3)])
+    batch = builder.scenes_batch([scenes.pyramid(5 + k) for k in range(3)])
     batch.world_i[:, L.WI_FLAGS] |= L.WF_CUSTOM_FILTER
     e = N.Engine("fp64")
     e.upload(batch)
