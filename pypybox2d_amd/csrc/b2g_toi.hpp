@@ -26,8 +26,9 @@ constexpr double kToiPi = 3.141592653589793;
 enum : int { TOI_UNKNOWN = 0, TOI_FAILED, TOI_OVERLAPPED, TOI_TOUCHING, TOI_SEPARATED, TOI_STUCK };
 
 // DistanceProxy (distance.py:355-400): a circle's centre, a polygon's vertices, an edge's ends.
+// The vertices' memory is the caller's (B2G_MAX_POLY_VERTS of them).
 struct TProxy {
-  V2<double> v[8];
+  V2<double>* v;
   int n;
   double radius;
 };
