@@ -4523,6 +4523,7 @@ struct ToiScratch {
   VC<double> vc[kToiContacts];
   ToiPC pc[kToiContacts];
   ToiPV pv[kToiBodies];
+  RotMemo rot[kToiBodies];  // of pv's angles
   int bodies[kToiBodies];
   int contacts[kToiContacts];
 };
@@ -4568,11 +4569,12 @@ __device__ inline bool toi_position_sweep(ToiScratch& S, int nc) {
     const ToiPC& pc = S.pc[k];
     V2<double> ca = S.pv[pc.ia].c, cb = S.pv[pc.ib].c;
     double aa = S.pv[pc.ia].a, ab = S.pv[pc.ib].a;
+    RotMemo qa = S.rot[pc.ia], qb = S.rot[pc.ib];
     const bool mva = pc.ia < 2, mvb = pc.ib < 2;
     const double ima = mva ? pc.ma : 0.0, iIa = mva ? pc.Ia : 0.0;
     const double imb = mvb ? pc.mb : 0.0, iIb = mvb ? pc.Ib : 0.0;
     for (int j = 0; j < pc.npts; ++j) {
-      const XF<double> xfa = xf_at(ca, aa, pc.lca), xfb = xf_at(cb, ab, pc.lcb);
+      const XF<double> xfa = xf_with(ca, qa.at(aa), pc.lca), xfb = xf_with(cb, qb.at(ab), pc.lcb);
       V2<double> normal, point;
       double sep;
       const V2<double> lpj = j == 0 ? pc.lp0 : pc.lp1;
@@ -4609,6 +4611,8 @@ __device__ inline bool toi_position_sweep(ToiScratch& S, int nc) {
     S.pv[pc.ia].a = aa;
     S.pv[pc.ib].c = cb;
     S.pv[pc.ib].a = ab;
+    S.rot[pc.ia] = qa;
+    S.rot[pc.ib] = qb;
   }
   return min_sep >= -1.5 * LINEAR_SLOP;
 }
@@ -4876,6 +4880,7 @@ __device__ void world_solve_toi(const Dev<T>& d, int w, ToiLds& L) {
       const double2 c = d.b_c[gb];
       S.pv[i].c = v2<double>(c.x, c.y);
       S.pv[i].a = d.b_a[gb];
+      S.rot[i].set(S.pv[i].a);
       S.pv[i].v = d.b_v[gb];
       S.pv[i].w = d.b_w[gb];
     }

@@ -255,16 +255,32 @@ struct TSweep {
   double a0, a, alpha0;
 };
 
-__device__ inline XF<double> xf_at(V2<double> c, double a, V2<double> lc) {
+__device__ inline XF<double> xf_with(V2<double> c, Rot<double> q, V2<double> lc) {
   XF<double> t;
-  t.q = rot_of<double>(a);
+  t.q = q;
   t.p = c - rmul(t.q, lc);
   return t;
 }
+__device__ inline XF<double> xf_at(V2<double> c, double a, V2<double> lc) { return xf_with(c, rot_of<double>(a), lc); }
 
-__device__ inline XF<double> sweep_xf(const TSweep& s, double beta) {  // Sweep.get_transform
+// The rotation of the last angle asked for.  A sine and cosine cost about as much as the rest of a
+// separation or a position constraint, and a body that does not turn asks for the same angle again.
+struct RotMemo {
+  double a;
+  Rot<double> q;
+  __device__ inline void set(double angle) {
+    a = angle;
+    q = rot_of<double>(a);
+  }
+  __device__ inline Rot<double> at(double angle) {
+    if (__double_as_longlong(angle) != __double_as_longlong(a)) set(angle);
+    return q;
+  }
+};
+
+__device__ inline XF<double> sweep_xf(const TSweep& s, double beta, RotMemo& m) {  // Sweep.get_transform
   const V2<double> p = scale(1.0 - beta, s.c0) + scale(beta, s.c);
-  return xf_at(p, (1.0 - beta) * s.a0 + beta * s.a, s.lc);
+  return xf_with(p, m.at((1.0 - beta) * s.a0 + beta * s.a), s.lc);
 }
 
 __device__ inline void sweep_advance(TSweep& s, double alpha) {  // Sweep.advance
@@ -279,12 +295,13 @@ struct SepFn {
   const TProxy* pa;
   const TProxy* pb;
   TSweep sa, sb;
+  RotMemo ma, mb;
   int type;
   V2<double> axis, lp;
 };
 
 __device__ inline void sep_init(SepFn& f, const GjkCache& cache, double t1) {  // toi.py:54-122
-  const XF<double> xfa = sweep_xf(f.sa, t1), xfb = sweep_xf(f.sb, t1);
+  const XF<double> xfa = sweep_xf(f.sa, t1, f.ma), xfb = sweep_xf(f.sb, t1, f.mb);
   const int ia0 = cache.ia[0], ib0 = cache.ib[0];
   if (cache.count == 1) {
     f.type = SEP_POINTS;
@@ -312,8 +329,8 @@ __device__ inline void sep_init(SepFn& f, const GjkCache& cache, double t1) {  /
 }
 
 // find_min_separation (find = true; toi.py:124-175) or evaluate (toi.py:177-213)
-__device__ inline double sep_eval(const SepFn& f, bool find, int& ia, int& ib, double t) {
-  const XF<double> xfa = sweep_xf(f.sa, t), xfb = sweep_xf(f.sb, t);
+__device__ inline double sep_eval(SepFn& f, bool find, int& ia, int& ib, double t) {
+  const XF<double> xfa = sweep_xf(f.sa, t, f.ma), xfb = sweep_xf(f.sb, t, f.mb);
   if (f.type == SEP_POINTS) {
     if (find) {
       ia = tproxy_support(*f.pa, rmul_t(xfa.q, f.axis));
@@ -352,6 +369,8 @@ __device__ inline int time_of_impact(const TProxy& pa, const TProxy& pb, const T
   d = 2.0 * kToiPi * floor(f.sb.a0 / (2.0 * kToiPi));
   f.sb.a0 -= d;
   f.sb.a -= d;
+  f.ma.set(f.sa.a0);
+  f.mb.set(f.sb.a0);
   const double total_radius = pa.radius + pb.radius;
   const double target = pmax(kToiLinearSlop, total_radius - 3.0 * kToiLinearSlop);
   const double tolerance = 0.25 * kToiLinearSlop;
@@ -361,7 +380,7 @@ __device__ inline int time_of_impact(const TProxy& pa, const TProxy& pb, const T
   cache.count = 0;
   cache.metric = 0.0;
   for (;;) {
-    const XF<double> xfa = sweep_xf(f.sa, t1), xfb = sweep_xf(f.sb, t1);
+    const XF<double> xfa = sweep_xf(f.sa, t1, f.ma), xfb = sweep_xf(f.sb, t1, f.mb);
     const double dist = gjk_distance(pa, pb, xfa, xfb, cache);
     if (dist <= 0.0) {
       state = TOI_OVERLAPPED;
