@@ -108,6 +108,8 @@ __host__ __device__ inline int size_class(int nc) {  // floor(log2(nc + 1)), cap
 }
 
 constexpr int kSolveBlock = 64;  // k_solve: one wavefront per workgroup
+constexpr int kJointLdsMax = 65536;   // most LDS of a joint island (k_solve_joints_lds)
+constexpr int kCus = 256;             // compute units
 constexpr int kGroupBlock = 512;      // k_solve_group: eight wavefronts
 constexpr int kGroupWaves = kGroupBlock / 64;
 constexpr int kGroupPolls = 1 << 22;  // polls of a dataflow without its end: WERR_SCHEDULE
@@ -715,6 +717,11 @@ __device__ __forceinline__ int wave_same(int v) {
 }
 __device__ __forceinline__ bool wave_any(bool p) {
   return __ballot(p) != 0;
+}
+template <typename X>
+__device__ __forceinline__ X team_min(X v, int T) {
+  for (int off = T >> 1; off > 0; off >>= 1) v = pmin(v, (X)__shfl_xor(v, off, T));
+  return v;
 }
 struct IslandSmem {
   int* off;        // nb + 1
@@ -2168,6 +2175,100 @@ __device__ void solve_island_joints(const Dev<T>& d, int w, int bstart, int nbi,
   }
 }
 
+// The same by a wavefront with the island's joint records, their bodies' constants and the body
+// states in LDS.  The sweeps stay with lane 0 (joints and contacts in their order, each a chain of
+// reads and writes of the records); the lanes share the copies and what is independent per body.
+struct JointLds {
+  double rec[B2G_JOINT_ND];
+  JBodies bodies;
+  int irec[B2G_JOINT_NI];
+};
+static_assert(sizeof(JointLds) % 8 == 0, "JointLds");
+__host__ __device__ inline size_t joint_lds_bytes(int joints, int bodies) {
+  return (size_t)joints * sizeof(JointLds) + (size_t)bodies * sizeof(PV<double>);
+}
+
+template <typename T>
+__device__ __forceinline__ void solve_island_joints_lds(const Dev<T>& dg, int w, int bstart, int nbi, int cstart,
+                                                        int nci, int last_allow, char* lds, SolveMarks& mk) {
+  const IslandK c = island_k(dg, w, bstart);
+  const int lane = threadIdx.x;
+  const int2 jr = dg.i_jr[bstart];
+  const int je = jr.x, nje = jr.y, j0 = dg.w_joint_off[w];
+  JointLds* jl = (JointLds*)lds;
+  PV<T>* pv = (PV<T>*)(jl + nje);
+  for (int i = lane; i < nbi; i += 64) pv[i] = dg.pv[bstart + i];
+  for (int k = lane; k < nje; k += 64) {
+    const JRec J = island_joint(dg, c.b0, j0, je + k, jl[k].bodies);
+    for (int q = 0; q < B2G_JOINT_NI; ++q) jl[k].irec[q] = J.i[q];
+  }
+  for (int x = lane; x < nje * B2G_JOINT_ND; x += 64) {
+    const int k = x / B2G_JOINT_ND, q = x % B2G_JOINT_ND;
+    jl[k].rec[q] = dg.j_d[(size_t)(j0 + dg.i_joints[je + k]) * B2G_JOINT_ND + q];
+  }
+  Dev<T> d = dg;  // the sweeps' view: the island's body states in LDS
+  d.pv = pv;  // (from entry 0 on)
+  const IslandIO<T> io{&d, 0, c.b0};
+  JStep jst;
+  jst.dt = c.dt;
+  jst.inv_dt = d.inv_dt;
+  jst.dt_ratio = c.dt_ratio;
+  jst.warm = c.warm;
+  team_sync();
+  if (lane == 0) {
+    if (c.warm) velocity_sweep<T, true>(d, 0, cstart, nci);
+    for (int k = 0; k < nje; ++k)
+      if (!joint_init(JRec{jl[k].rec, jl[k].irec}, jl[k].bodies, io, jst)) atomicOr(&d.w_err[w], WERR_JOINT);
+    for (int it = 0; it < d.vel_iters; ++it) {
+      for (int k = 0; k < nje; ++k) joint_solve_velocity(JRec{jl[k].rec, jl[k].irec}, jl[k].bodies, io, jst);
+      velocity_sweep<T, false>(d, 0, cstart, nci);
+    }
+  }
+  if (d.i_time) mk.t_vel = (long long)wall_clock64();
+  team_sync();
+  for (int k = lane; k < nci; k += 64) store_impulse(d, c, cstart, k, d.vc[cstart + k]);
+  for (int i = lane; i < nbi; i += 64) {
+    PV<T> p = pv[i];
+    integrate_position(p, c.dt);
+    pv[i] = p;
+  }
+  team_sync();
+  int solved = 0, npos = 0;  // lane 0's
+  if (lane == 0)
+    for (int it = 0; it < d.pos_iters; ++it) {
+      npos = it + 1;
+      const bool contacts_okay = position_sweep(d, 0, cstart, nci);
+      bool joints_okay = true;
+      for (int k = 0; k < nje; ++k) {
+        const bool ok = joint_solve_position(JRec{jl[k].rec, jl[k].irec}, jl[k].bodies, io);
+        joints_okay = joints_okay && ok;
+      }
+      if (contacts_okay && joints_okay) {
+        solved = 1;
+        break;
+      }
+    }
+  mk.npos = wave_same(npos);
+  const bool position_solved = wave_same(solved) != 0;
+  team_sync();
+  for (int i = lane; i < nbi; i += 64) write_back(d, c, bstart, i, pv[i]);
+  for (int x = lane; x < nje * B2G_JOINT_ND; x += 64) {
+    const int k = x / B2G_JOINT_ND, q = x % B2G_JOINT_ND;
+    d.j_d[(size_t)(j0 + d.i_joints[je + k]) * B2G_JOINT_ND + q] = jl[k].rec[q];
+  }
+  for (int x = lane; x < nje * B2G_JOINT_NI; x += 64) {
+    const int k = x / B2G_JOINT_NI, q = x % B2G_JOINT_NI;
+    d.j_i[(size_t)(j0 + d.i_joints[je + k]) * B2G_JOINT_NI + q] = jl[k].irec[q];
+  }
+  if (c.wflags & WF_ALLOW_SLEEP) {  // (each lane reads back only the bodies it wrote)
+    double min_sleep = 1.0e300;
+    for (int i = lane; i < nbi; i += 64) min_sleep = pmin(min_sleep, sleep_body(d, c, bstart, i, last_allow));
+    min_sleep = team_min(min_sleep, 64);
+    if (min_sleep >= TIME_TO_SLEEP && position_solved && nbi > 0 && lane == (nbi - 1) % 64)
+      sleep_last(d, c, bstart, nbi);
+  }
+}
+
 // Island.solve on one lane (island.py:65-179).
 template <typename T>
 __device__ void solve_island(const Dev<T>& d, int w, int bstart, int nbi, int cstart, int nci, int last_allow,
@@ -2230,11 +2331,6 @@ __device__ __forceinline__ bool island_has_joints(const Dev<T>& d, int w, int bs
 // is the same code as the one-lane path, so results are identical.
 // ---------------------------------------------------------------------------
 
-template <typename X>
-__device__ __forceinline__ X team_min(X v, int T) {
-  for (int off = T >> 1; off > 0; off >>= 1) v = pmin(v, (X)__shfl_xor(v, off, T));
-  return v;
-}
 
 template <typename T>
 __device__ void solve_island_team(const Dev<T>& d, int w, int bstart, int nbi, int cstart, int nci, int last_allow,
@@ -2955,9 +3051,12 @@ __global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_e
   }
 }
 
-// The islands with joints, one lane each, after k_solve (which leaves them): launched only for
+// The islands with joints, after k_solve (which leaves them): launched only for
 // batches with joints.  Their bodies and contacts belong to no other island, so the order of the
-// two kernels does not matter.
+// two kernels does not matter.  k_solve_joints takes them a lane each, k_solve_joints_lds a
+// wavefront each where every world's joints and bodies fit its LDS.  Bound by the serial sweeps' reads: the testbed's bridge
+// (31 joints) takes 357 us a lane with its records in HBM and about 290 us in LDS.  Batches of more
+// worlds with joints than fit the chip's LDS side by side take the lanes, 64 islands a wavefront.
 template <typename T>
 __global__ void __launch_bounds__(64) k_solve_joints(Dev<T> d) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2970,6 +3069,23 @@ __global__ void __launch_bounds__(64) k_solve_joints(Dev<T> d) {
   SolveMarks mk{0, 0};
   solve_island_joints(d, in.x, in.y, nbi, in.w, nci, (nc >> 30) & 1, mk);
   if (d.i_time) record_island_time(d, q, t0, nci, nbi, 0, (int)((uint32_t)in.z >> 16), mk);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64) k_solve_joints_lds(Dev<T> d) {
+  extern __shared__ __align__(16) char joint_lds[];
+  const int n = *d.q_count;
+  for (int q = blockIdx.x; q < n; q += gridDim.x) {
+    const int4 in = d.qs_isl[q];
+    if (!island_has_joints(d, in.x, in.y)) continue;
+    const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
+    const int nc = d.qs_nc[q];
+    const int nbi = in.z & 0xFFFF, nci = nc & 0x3FFFFFFF;
+    SolveMarks mk{0, 0};
+    solve_island_joints_lds(d, in.x, in.y, nbi, in.w, nci, (nc >> 30) & 1, joint_lds, mk);
+    if (d.i_time && threadIdx.x == 0) record_island_time(d, q, t0, nci, nbi, 0, (int)((uint32_t)in.z >> 16), mk);
+    team_sync();  // the next island reuses the LDS
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -5866,6 +5982,7 @@ struct b2g_ctx {
   int* xbuf = nullptr;          // argument and result staging of the between-step calls
   size_t xcap = 0;              // ints in xbuf
   int nj = 0;                   // joints of the batch
+  int joint_lds = 0;            // LDS of k_solve_joints_lds; 0: k_solve_joints
   // readout: pinned host memory (the status of the last sync, the records' staging) and device
   // scratch made by the first download of a batch
   Status* status = nullptr;
@@ -6013,6 +6130,8 @@ static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
     }
   }
   HIPCHK(hipFuncSetAttribute((const void*)k_solve<T>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+  HIPCHK(hipFuncSetAttribute((const void*)k_solve_joints_lds<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             kJointLdsMax));
   HIPCHK(hipFuncSetAttribute((const void*)k_tree_build<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)(kTreeLdsKeys * sizeof(unsigned long long))));
 
@@ -6317,7 +6436,7 @@ static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
   }
   // joints: their records, each body's joint list (Body.joints, world.py:268-273), and the body
   // pairs a joint keeps from colliding (body.py:920-926)
-  ctx->nj = 0;
+  ctx->nj = ctx->joint_lds = 0;
   if (b->joint_off && b->joint_off[nw] > 0) {
     const int nj = b->joint_off[nw];
     if (!b->joint_d || !b->joint_i) return set_error(ctx, B2G_E_INVALID, "joint records missing");
@@ -6406,6 +6525,16 @@ static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
     d.w_jnc_off = wjn;
     d.jnc = jncd;
     ctx->nj = nj;
+    int joint_worlds = 0;
+    size_t need = 0;  // the largest island a world's joints and bodies can make
+    for (int w = 0; w < nw; ++w) {
+      const int k = b->joint_off[w + 1] - b->joint_off[w];
+      if (k == 0) continue;
+      ++joint_worlds;
+      need = std::max(need, joint_lds_bytes(k, b->body_off[w + 1] - b->body_off[w]));
+    }
+    need = (need + 255) & ~(size_t)255;
+    if (need <= (size_t)kJointLdsMax && joint_worlds <= kCus * (kMaxLds / (int)need)) ctx->joint_lds = (int)need;
   }
   if (!ctx->big.empty()) {  // scratch of the large-world path
     int *wb = nullptr, *bl = nullptr;
@@ -6663,7 +6792,10 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
       HIPCHK(hipEventRecord(ctx->join_ev[0], ctx->aux[0]));
       HIPCHK(hipStreamWaitEvent(st, ctx->join_ev[0], 0));
     }
-    if (ctx->nj > 0)
+    if (ctx->joint_lds > 0)
+      hipLaunchKernelGGL(k_solve_joints_lds<T>, dim3((unsigned)std::max(1, std::min(ctx->nb, 4096))), dim3(64),
+                         (size_t)ctx->joint_lds, st, d);
+    else if (ctx->nj > 0)
       hipLaunchKernelGGL(k_solve_joints<T>, dim3((unsigned)std::max(1, (ctx->nb + 63) / 64)), dim3(64), 0, st, d);
     if (part == PART_ISLANDS) {
       HIPCHK(hipGetLastError());
