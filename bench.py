@@ -192,7 +192,7 @@ def run_gpu(start: L.BatchArrays, precision: str, steps: int, warmup: int, tune:
 def solver_report(rows: np.ndarray, waves_per_cu: int) -> dict:
     """The island solver as occupancy plus per-island latency (it is bound by the dependency
     chains inside islands, not by bytes): one step's islands grouped by the lanes that solved
-    them (a team's size; 1: one lane per island; 0: a team island solved by one lane)."""
+    them (a team's size; 64 also: a group of wavefronts; 1: one lane per island; 0: a team island solved by one lane)."""
     start, end = rows[:, 0], rows[:, 1]
     lat = (end - start) / 1e3
     span = (end.max() - start.min()) / 1e3
@@ -418,7 +418,7 @@ def roofline(stage: str, ms: float, c: dict, w: dict, fp64: bool, args) -> dict:
 LATENCY_LIMITS = {
     "k_solve": "dependency chains inside the largest islands: passes (about the Gauss-Seidel dependency depth "
                "of all sweeps) x pass latency; see the solver report (occupancy and per-island latency)",
-    "k_islands": "one lane walks each world's (or island's) depth-first search",
+    "k_islands": "one wavefront walks each world's contact graph depth-first",
 }
 
 
