@@ -725,7 +725,7 @@ __device__ __forceinline__ X team_min(X v, int T) {
 }
 struct IslandSmem {
   int* off;        // nb + 1
-  int* cur;        // nb
+  int* cur;        // nb; in the end, at each island's start in the island-body list, its sweep period
   uint32_t* adj;    // adjacency entries: contact slot | other body << 16
   uint8_t* bst;    // nb: bit0 static, bit1 awake, bit2 allow_sleep, bit3 active, bit4 flag, bit5 woken,
                    // bit6 touches some body more than once
@@ -733,9 +733,8 @@ struct IslandSmem {
   uint16_t* stack;  // nb
   uint16_t* slist;  // nb: the static bodies of an island; then, per place in the island-body list, the
                     // first contact its body takes
-  uint16_t* lev;    // nb: dependency level of the body's first contact in the island list
+  uint16_t* lev;    // nb: dependency level of the body's first contact, then the sweep period it asks for
   uint16_t* ibs;    // nb: start of the body's island in the island-body list
-  int* per;         // nb: per island, at its start in the island-body list, its sweep period
   int* scan;       // kBlock
   int* misc;       // 8
 };
@@ -768,7 +767,8 @@ __host__ __device__ inline size_t island_smem_bytes(int nb, int nf, int ccap) {
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;  // lev
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;  // ibs
-  s += ((size_t)nb * 4 + 15) & ~(size_t)15;  // per
+  // free: a bit per contact slot, so that the same worlds fit whose joints the other path refuses
+  s += ((size_t)(ccap + 31) / 32 * 4 + 15) & ~(size_t)15;
   s += (size_t)kBlock * 4;
   s += 64 * 4;  // misc: 16 scalars, 16 class counts, spare
   return s;
@@ -829,7 +829,6 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
     L.slist = (uint16_t*)p; p += ((size_t)nb * 2 + 15) & ~(size_t)15;
     L.lev = (uint16_t*)p; p += ((size_t)nb * 2 + 15) & ~(size_t)15;
     L.ibs = (uint16_t*)p; p += ((size_t)nb * 2 + 15) & ~(size_t)15;
-    L.per = (int*)p; p += ((size_t)nb * 4 + 15) & ~(size_t)15;
     L.scan = (int*)p; p += (size_t)kBlock * 4;
     L.misc = (int*)p;
   }
@@ -1156,10 +1155,7 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   // The contacts' dependency levels: one more than the latest level among their dynamic bodies'
   // contacts before them.  A lane polls its contacts in list order, which every dependency follows;
   // cur holds a body's contacts done << 16 | the last one's level.
-  for (int i = tid; i < nb; i += kBlock) {
-    L.cur[i] = 0;
-    L.per[i] = 1;
-  }
+  for (int i = tid; i < nb; i += kBlock) L.cur[i] = 0;
   for (int c = tid; c < nci_tot; c += kBlock) {  // (the lane's own records: no barrier between)
     const uint2 r = d.i_rank[cb + c];
     L.adj[2 * c] = r.x | d.i_order[cb + c] << 16;
@@ -1203,17 +1199,22 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
     }
   }
   __syncthreads();
+  // the islands' sweep periods: the largest that one of their bodies asks for, through lev into cur
   for (int b = tid; b < nb; b += kBlock) {
     const uint32_t wb = (uint32_t)L.cur[b];
-    if ((L.bst[b] & (1 | 16)) == 16 && wb)
-      atomicMax(&L.per[L.ibs[b]], sweep_period((int)(wb & 0xFFFFu) - (int)L.lev[b], (int)(wb & 0xFFFFu)));
+    L.lev[b] = wb ? (uint16_t)sweep_period((int)(wb & 0xFFFFu) - (int)L.lev[b], (int)(wb & 0xFFFFu)) : (uint16_t)0;
   }
+  __syncthreads();
+  for (int i = tid; i < nb; i += kBlock) L.cur[i] = 1;
+  __syncthreads();
+  for (int b = tid; b < nb; b += kBlock)
+    if ((L.bst[b] & (1 | 16)) == 16) atomicMax(&L.cur[L.ibs[b]], (int)L.lev[b]);
   __syncthreads();
   for (int k = tid; k < nisl; k += kBlock) {
     const int4 in = info[k];
     const int next = in.x + in.y, cstart = L.slist[in.x];
     const int nc = (next < nbi_tot ? (int)L.slist[next] : nci_tot) - cstart;
-    info[k] = make_int4(in.x, in.y | L.per[in.x] << 16, cstart, nc | in.w);
+    info[k] = make_int4(in.x, in.y | L.cur[in.x] << 16, cstart, nc | in.w);
   }
   // the island joints' bodies as island-local indices (a body outside the island's body list,
   // a static one, as -1 - world-local index)
