@@ -112,7 +112,13 @@ constexpr int kJointLdsMax = 65536;   // most LDS of a joint island (k_solve_joi
 constexpr int kCus = 256;             // compute units
 constexpr int kGroupBlock = 512;      // k_solve_group: eight wavefronts
 constexpr int kGroupWaves = kGroupBlock / 64;
-constexpr int kGroupPolls = 1 << 22;  // polls of a dataflow without its end: WERR_SCHEDULE
+// Polls of a dataflow of n solves without its end: WERR_SCHEDULE.  At least one solve is always ready, and a
+// poll in vain of one wavefront takes a tenth of a solve of another (some 150 cycles of 1500), so n
+// solves one after another, as of a body with n contacts, take some 10 n polls.
+__host__ __device__ inline int poll_limit(long long n) {
+  const long long p = 64 * n + (1 << 16);
+  return p < 0x7FFFFFFF ? (int)p : 0x7FFFFFFF;
+}
 constexpr int kGroupTopClass = 9;     // the largest islands with a lane per two contacts
 constexpr int kGroupLastClass = 5;     // groups take every island of this class and above, or none
 constexpr int kGroupMaxContacts = (1 << (kGroupTopClass + 1)) - 2;
@@ -1164,8 +1170,9 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   __syncthreads();
   {
     int c = tid, poll = 0;
+    const int polls = poll_limit(nci_tot);
     uint32_t who = c < nci_tot ? L.adj[2 * c] : 0u, rank = c < nci_tot ? L.adj[2 * c + 1] : 0u;
-    while (wave_any(c < nci_tot) && poll < kGroupPolls) {
+    while (wave_any(c < nci_tot) && poll < polls) {
       ++poll;
       const int b = (int)(who & 0xFFFFu), o = (int)(who >> 16);
       const uint32_t rb = rank & 0xFFFFu, ro = rank >> 16;
@@ -2875,7 +2882,8 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
     }
     group_sync(bar, due, waves);
     int poll = 0;
-    while (wave_any(pend) && poll < kGroupPolls) {
+    const int polls = poll_limit((long long)nsw * nci);
+    while (wave_any(pend) && poll < polls) {
       ++poll;
       pend = false;
 #pragma unroll
@@ -2928,6 +2936,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
       tb[j] = cur[j].rkb & 0xFFFF;
     }
     group_sync(bar, due, waves);
+    const int polls = poll_limit(nci);
     for (int it = 0; it < d.pos_iters && !position_solved; ++it) {  // group-uniform
       if (d.i_time) mk.npos = it + 1;
       T min_sep = 0;
@@ -2938,7 +2947,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
         pend |= has[j];
       }
       int poll = 0;
-      while (wave_any(pend) && poll < kGroupPolls) {
+      while (wave_any(pend) && poll < polls) {
         ++poll;
         pend = false;
 #pragma unroll

@@ -6,6 +6,7 @@ import pytest
 
 from pypybox2d_amd import _native as N
 from pypybox2d_amd import builder, layout as L, scenes
+from pypybox2d_amd.scenes import _body, _fix
 
 pytestmark = pytest.mark.gpu
 DT = 1.0 / 60
@@ -66,3 +67,28 @@ def test_piles_static_sides_and_iteration_counts(prec, iters):
     e.close()
     state.world_i[::2, L.WI_FLAGS] &= ~L.WF_WARM_STARTING
     _run(prec, state, *iters)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_many_iterations_on_a_body_of_many_contacts(prec):
+    """Each of a slab's 301 contacts waits for the one before it: 4001 sweeps are 1.2 million solves one
+    after another, and the poll limit has to grow with them."""
+    bodies = [_body("static", (0.0, 0.0), [_fix(("edge", (-600.0, 0.0), (600.0, 0.0)))]),
+              _body("dynamic", (0.0, 0.5), [_fix(("box", 180.0, 0.5), density=2.0, friction=0.5)])]
+    bodies += [_body("dynamic", (1.1 * (k - 149.5), 1.49), [_fix(("box", 0.5, 0.5), density=1.0, friction=0.5)])
+               for k in range(300)]
+    batch = builder.scene_batch({"gravity": (0.0, -10.0), "bodies": bodies, "do_sleep": False, "warm_starting": True})
+    out = []
+    for load in (1 << 20, 0):
+        e = N.Engine(prec)
+        e.set_param("group_load", load)
+        e.set_param("island_times", 1)
+        e.upload(batch)
+        e.step_n(3, DT, 8, 3, graph=True)
+        e.step(DT, 4000, 3)
+        out.append((e.download(), e.island_times()))
+        print(prec, load, "done", flush=True)
+        e.close()
+    assert out[0][1][0, 2] >= 300 and out[0][1][0, 4] == 64 and 1 < out[1][1][0, 4] < 64
+    for f in ("body_d", "con_d", "con_i"):
+        assert np.array_equal(getattr(out[0][0], f), getattr(out[1][0], f)), f
