@@ -724,6 +724,19 @@ __device__ __forceinline__ int wave_same(int v) {
 __device__ __forceinline__ bool wave_any(bool p) {
   return __ballot(p) != 0;
 }
+// The end of a poll, with and without success, in a loop whose lanes wait for one another.  A lane
+// that has its turn must not wait for the others of its wavefront to have theirs: were the loop
+// entered again with the same state straight from a poll in vain, the compiler would make those polls
+// a loop of their own, which the wavefront leaves only as a whole, and a lane that waits for another
+// one there waits for ever.  So both outcomes meet here, and the state is new in every pass.
+template <typename X>
+__device__ __forceinline__ void made_new(X& v) {
+  asm volatile("" : "+v"(v));
+}
+template <typename... X>
+__device__ __forceinline__ void poll_end(X&... state) {
+  (made_new(state), ...);
+}
 template <typename X>
 __device__ __forceinline__ X team_min(X v, int T) {
   for (int off = T >> 1; off > 0; off >>= 1) v = pmin(v, (X)__shfl_xor(v, off, T));
@@ -1194,11 +1207,7 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
         who = L.adj[2 * n];
         rank = L.adj[2 * n + 1];
       }
-      // A lane that has its turn must not wait for the others of its wavefront to have theirs: were
-      // its state the same after a poll in vain, the compiler would make those polls a loop of their
-      // own, which the wavefront leaves only as a whole, and a lane that waits for another one there
-      // waits for ever.  So the state is made new in every pass.
-      asm volatile("" : "+v"(c), "+v"(who), "+v"(rank));
+      poll_end(c, who, rank);
     }
     if (c < nci_tot) {  // poll limit reached: any level, so that what follows stays in range
       atomicOr(&d.w_err[w], WERR_SCHEDULE);
@@ -2900,6 +2909,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
           tb[j] += (int)((unsigned)cur[j].rkb >> 16);
           --left[j];
         }
+        poll_end(ta[j], tb[j]);
         pend |= left[j] > 0;
       }
     }
@@ -2964,6 +2974,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
             tb[j] += (int)((unsigned)cur[j].rkb >> 16);
             todo[j] = false;
           }
+          poll_end(ta[j], tb[j]);
           pend |= todo[j];
         }
       }
