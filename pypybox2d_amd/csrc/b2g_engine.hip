@@ -112,16 +112,18 @@ constexpr int kJointLdsMax = 65536;   // most LDS of a joint island (k_solve_joi
 constexpr int kCus = 256;             // compute units
 constexpr int kGroupBlock = 512;      // k_solve_group: eight wavefronts
 constexpr int kGroupWaves = kGroupBlock / 64;
-// Polls of a dataflow of n solves without its end: WERR_SCHEDULE.  At least one solve is always ready, and a
-// poll in vain of one wavefront takes a tenth of a solve of another (some 150 cycles of 1500), so n
-// solves one after another, as of a body with n contacts, take some 10 n polls.
-__host__ __device__ inline int poll_limit(long long n) {
-  const long long p = 64 * n + (1 << 16);
-  return p < 0x7FFFFFFF ? (int)p : 0x7FFFFFFF;
-}
+// Polls of a dataflow without its end: WERR_SCHEDULE.  At least one solve is always ready, and a poll in
+// vain of one wavefront takes a tenth of a solve of another (some 150 cycles of 1500): n solves one
+// after another, as of a body with n contacts, take up to kSolvePolls n polls.  The limit is a constant, since a
+// limit of its own for each island, however held, costs the solve stage 2 to 4 %; steps of so many
+// iterations that an island could reach it (groups_allowed) are left to k_solve.
+constexpr int kGroupPolls = 1 << 26;
+constexpr int kSolvePolls = 16;
 constexpr int kGroupTopClass = 9;     // the largest islands with a lane per two contacts
 constexpr int kGroupLastClass = 5;     // groups take every island of this class and above, or none
 constexpr int kGroupMaxContacts = (1 << (kGroupTopClass + 1)) - 2;
+// May islands be solved by groups in a step of these iterations (up to 4103)?
+inline bool groups_allowed(int vel_iters) { return (vel_iters + 1ll) * kGroupMaxContacts * kSolvePolls <= kGroupPolls; }
 
 // Wavefronts of an island of a group class: a lane per contact up to class 8 (510 contacts).
 __host__ __device__ inline int group_waves(int cls) {
@@ -1183,9 +1185,8 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   __syncthreads();
   {
     int c = tid, poll = 0;
-    const int polls = poll_limit(nci_tot);
     uint32_t who = c < nci_tot ? L.adj[2 * c] : 0u, rank = c < nci_tot ? L.adj[2 * c + 1] : 0u;
-    while (wave_any(c < nci_tot) && poll < polls) {
+    while (wave_any(c < nci_tot) && poll < kGroupPolls) {  // (fewer than 65535 contacts, a level each)
       ++poll;
       const int b = (int)(who & 0xFFFFu), o = (int)(who >> 16);
       const uint32_t rb = rank & 0xFFFFu, ro = rank >> 16;
@@ -2891,8 +2892,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
     }
     group_sync(bar, due, waves);
     int poll = 0;
-    const int polls = poll_limit((long long)nsw * nci);
-    while (wave_any(pend) && poll < polls) {
+    while (wave_any(pend) && poll < kGroupPolls) {
       ++poll;
       pend = false;
 #pragma unroll
@@ -2946,7 +2946,6 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
       tb[j] = cur[j].rkb & 0xFFFF;
     }
     group_sync(bar, due, waves);
-    const int polls = poll_limit(nci);
     for (int it = 0; it < d.pos_iters && !position_solved; ++it) {  // group-uniform
       if (d.i_time) mk.npos = it + 1;
       T min_sep = 0;
@@ -2957,7 +2956,7 @@ __device__ __forceinline__ void solve_island_group(const Dev<T>& d, int w, int b
         pend |= has[j];
       }
       int poll = 0;
-      while (wave_any(pend) && poll < polls) {
+      while (wave_any(pend) && poll < kGroupPolls) {
         ++poll;
         pend = false;
 #pragma unroll
@@ -6700,7 +6699,7 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
   d.vel_iters = vi;
   d.pos_iters = pi;
   d.heavy_class = ctx->heavy_class;
-  d.group_load = ctx->group_load;
+  d.group_load = groups_allowed(vi) ? ctx->group_load : 0;
   d.team_full_class = ctx->team_full_class;
   d.team_lds = ctx->team_lds;
   d.team_max = ctx->team_max;
@@ -6799,13 +6798,13 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
     hipLaunchKernelGGL(k_prep_contacts<T>, dim3((unsigned)kPrepGrid), dim3(kBlock), 0, st, d);
     const int swaves = std::max(1, std::min((ctx->nb + kSolveBlock - 1) / kSolveBlock, ctx->solve_grid));
     // k_solve has work beside the groups' only in worlds that can hold an island too large for them
-    const bool beside = ctx->group_load > 0 && ctx->max_ccap > kGroupMaxContacts;
+    const bool beside = d.group_load > 0 && ctx->max_ccap > kGroupMaxContacts;
     if (beside) {
       HIPCHK(hipEventRecord(ctx->fork_ev, st));
       HIPCHK(hipStreamWaitEvent(ctx->aux[0], ctx->fork_ev, 0));
     }
     hipLaunchKernelGGL(k_solve<T>, dim3(swaves), dim3(kSolveBlock), ctx->team_lds, beside ? ctx->aux[0] : st, d);
-    if (ctx->group_load > 0) {
+    if (d.group_load > 0) {
       const int ggrid = std::max(1, std::min(ctx->nb, 4096));
       hipLaunchKernelGGL(k_solve_group<T>, dim3(ggrid), dim3(kGroupBlock), 0, st, d);
     }
