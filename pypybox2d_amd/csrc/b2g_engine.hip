@@ -35,7 +35,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <tuple>
 #include <vector>
@@ -6866,25 +6865,21 @@ static void launch_status(b2g_ctx* ctx) {
                      (const int*)d.w_con_used, (const int*)d.w_nisl, ctx->status);
 }
 
-// [0, n) cut into pieces for up to kCopyThreads threads: fn(begin, end).
+// [0, n) cut into pieces for up to kCopyThreads threads: fn(begin, end), which must not throw.
 constexpr int kCopyThreads = 8;
 template <typename F>
 static void host_parallel(size_t n, size_t grain, F fn) {
   const size_t want = std::min<size_t>(kCopyThreads, n / std::max<size_t>(grain, 1));
-  std::vector<std::thread> th;
+  std::thread th[kCopyThreads];
+  int started = 0;
   size_t done = 0;
-  if (want > 1) {
-    const size_t per = n / want;
-    try {
-      for (size_t k = 0; k + 1 < want; ++k) {
-        th.emplace_back(fn, done, done + per);
-        done += per;
-      }
-    } catch (const std::system_error&) {  // no thread to be had: this one does the rest
-    }
+  try {
+    for (const size_t per = n / std::max<size_t>(want, 1); (size_t)started + 1 < want; ++started, done += per)
+      th[started] = std::thread(fn, done, done + per);
+  } catch (...) {  // no thread to be had, or no memory for one: this one does the rest
   }
   fn(done, n);
-  for (auto& t : th) t.join();
+  for (int k = 0; k < started; ++k) th[k].join();
 }
 constexpr size_t kCopyGrain = (size_t)2 << 20;  // bytes a copying thread is worth
 static void host_copy(void* dst, const void* src, size_t bytes) {

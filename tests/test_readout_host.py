@@ -1,5 +1,11 @@
 """Host side of the readout: the pool of large arrays and the stepper's replay start."""
+import os
+import shutil
+import subprocess
+import sys
+
 import numpy as np
+import pytest
 
 from pypybox2d_amd import layout as L
 from pypybox2d_amd._native import host_copy
@@ -32,6 +38,49 @@ def test_threaded_copy_copies_every_byte():
         assert np.array_equal(host_copy(src, np.zeros(n)), src)
     src = np.arange(24.0).reshape(4, 6)
     assert np.array_equal(host_copy(src[:, ::2], np.zeros((4, 3))), src[:, ::2])
+
+
+NEW_FAILS = r"""
+#include <cstdlib>
+#include <new>
+extern "C" { long new_fails_at = -1; }
+void* operator new(std::size_t n) {
+  if (new_fails_at >= 0 && new_fails_at-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+"""
+
+COPY = r"""
+import ctypes, sys
+import numpy as np
+from pypybox2d_amd._native import host_copy, load
+load()
+fails = ctypes.c_long.in_dll(ctypes.CDLL(sys.argv[1]), "new_fails_at")
+src = np.arange(4_000_001, dtype=np.float64)
+for at in range(12):
+    fails.value = at
+    out = host_copy(src, np.zeros_like(src))
+    fails.value = -1
+    assert np.array_equal(out, src), at
+print("copied")
+"""
+
+
+def test_threaded_copy_without_memory_for_its_threads(tmp_path):
+    """An allocation that fails while the copying threads start: no exception leaves the C entry and no
+    running thread is dropped (either would end the process)."""
+    if not shutil.which("g++"):
+        pytest.skip("no C++ compiler")
+    (tmp_path / "n.cpp").write_text(NEW_FAILS)
+    lib = str(tmp_path / "libn.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", lib, str(tmp_path / "n.cpp")], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, LD_PRELOAD=" ".join(filter(None, [lib, os.environ.get("LD_PRELOAD")])))
+    r = subprocess.run([sys.executable, "-c", COPY, lib], cwd=root, env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "copied" in r.stdout, (r.returncode, r.stderr[-500:])
 
 
 class _Engine:
