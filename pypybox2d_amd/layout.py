@@ -288,15 +288,17 @@ class ArrayPool:
     def __init__(self):
         self._blocks: Dict[str, List[np.ndarray]] = {}
 
-    def get(self, name: str, shape, dtype) -> np.ndarray:
-        """An array with arbitrary contents."""
+    def get(self, name: str, shape, dtype, over: Optional[np.ndarray] = None) -> np.ndarray:
+        """An array with arbitrary contents: in the memory of ``over``, an array of this pool which the
+        caller alone refers to, where it fits (its contents stay until the new array is written)."""
         n = int(np.prod(shape))
         if n * np.dtype(dtype).itemsize < self.SMALL:
             return np.empty(shape, dtype)
         blocks = self._blocks.setdefault(name, [])
         for k in range(len(blocks)):
             # referred to by this list alone: no array made of it is left
-            if sys.getrefcount(blocks[k]) == 2 and n <= blocks[k].size <= 2 * n and blocks[k].dtype == dtype:
+            free = sys.getrefcount(blocks[k]) == 2 or (over is not None and over.base is blocks[k])
+            if free and n <= blocks[k].size <= 2 * n and blocks[k].dtype == dtype:
                 return blocks[k][:n].reshape(shape)
         block = np.empty(n + n // 16, dtype)
         blocks.append(block)

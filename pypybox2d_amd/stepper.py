@@ -70,19 +70,18 @@ class Stepper(object):
         if old is None or old.fix_d.shape != st.fix_d.shape:
             self._ckpt = st.copy()
             return
-        new = {}
+        new = {}  # all the memory first: if it cannot be had, the last start is still whole
         for n in L.ALL_FIELDS:
             src, out = getattr(st, n), getattr(old, n)
-            if n == "fix_d":
-                continue
-            if out.shape != src.shape:  # the contacts and moves of another frame
-                setattr(old, n, None)
-                out = None
-                out = self._pool.get(n, src.shape, src.dtype)
-            new[n] = host_copy(src, out)
+            # (the contacts and moves of another frame have another size)
+            new[n] = out if out.shape == src.shape else self._pool.get(n, src.shape, src.dtype, over=out)
         fat = slice(L.FD_FAT_LX, L.FD_FAT_LX + 4)
-        old.fix_d[:, fat] = st.fix_d[:, fat]
-        self._ckpt = L.BatchArrays(fix_d=old.fix_d, **new)
+        for n, out in new.items():
+            if n == "fix_d":
+                out[:, fat] = st.fix_d[:, fat]
+            else:
+                host_copy(getattr(st, n), out)
+        self._ckpt = L.BatchArrays(**new)
 
     def record(self, n: int, dt: float, vel_iters: int, pos_iters: int) -> None:
         """Logs n steps that were launched on the engine directly (e.g. by the launch tuner)."""

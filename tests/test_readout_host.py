@@ -30,6 +30,11 @@ def test_pool_never_hands_out_memory_that_is_still_referred_to():
     assert len({h.ctypes.data for h in held} | {b.ctypes.data, c.ctypes.data}) == 6
     assert len(pool._blocks["x"]) == 2  # bounded
     assert pool.get("x", shape, np.int32).dtype == np.int32
+    y = pool.get("y", shape, np.float64)
+    y[:] = 3.0
+    z = pool.get("y", (1900, 28), np.float64, over=y)  # the caller gives y up for it
+    assert z.ctypes.data == y.ctypes.data and np.all(z == 3.0)
+    assert pool.get("y", (5000, 28), np.float64, over=z).ctypes.data != z.ctypes.data
 
 
 def test_threaded_copy_copies_every_byte():
@@ -116,3 +121,23 @@ def test_replay_start_is_apart_from_the_state_given_out():
             getattr(st, f)[...] = -5
         for f in L.ALL_FIELDS:
             assert np.array_equal(getattr(s._ckpt, f), want[f]), (n, f)
+
+
+def test_replay_start_survives_a_readout_without_memory_for_its_own():
+    s = Stepper("fp32", 0, engine_factory=_Engine)
+    s.upload(_Engine().download())
+    s.download()
+    want = {f: getattr(s._ckpt, f).copy() for f in L.ALL_FIELDS}
+    s._log.append(("pairs",))
+
+    class Pool:
+        def get(self, name, shape, dtype, over=None):
+            if name == "con_i":
+                raise MemoryError(name)
+            return np.empty(shape, dtype)
+    s._pool = Pool()
+    with pytest.raises(MemoryError):
+        s.download()
+    for f in L.ALL_FIELDS:
+        assert np.array_equal(getattr(s._ckpt, f), want[f]), f
+    assert s._log == [("pairs",)]
