@@ -766,6 +766,10 @@ __device__ __forceinline__ size_t align16(size_t x) { return (x + 15) & ~(size_t
 // and reports a capacity error beyond that.  The adjacency arrays also hold
 // the awake-gating candidates, kGateChunk slots at a time.
 constexpr int kGateChunk = 1024;
+// Contacts of a body from which on a lane does not handle them alone.  The comparison of all pairs of a
+// body's entries by one lane took 11.6 ms of a slab under 600 boxes (0.55 ms of 600 boxes on static
+// ground); a wavefront for 64 entries, it takes 0.50 ms.
+constexpr int kHubContacts = 16;
 __host__ __device__ inline int touch_cap(int nf, int ccap) {
   const int t = 4 * nf + 64;
   return t < ccap ? t : ccap;
@@ -831,6 +835,7 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   constexpr int kBlock = B;
   extern __shared__ __align__(16) unsigned char smem[];
   const int w = d.w_order[w_first + blockIdx.x], tid = threadIdx.x;
+  const int lane = tid & 63, wv = tid >> 6;
   if (d.w_big && d.w_big[w]) return;  // k_islands_big
   const int b0 = d.w_body_off[w], nb = d.w_body_off[w + 1] - b0;
   const int f0 = d.w_fix_off[w], nf = d.w_fix_off[w + 1] - f0;
@@ -859,7 +864,7 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
                          ((fl & BF_ACTIVE) ? 8 : 0));
     L.off[i] = 0;
   }
-  if (tid == 0) L.misc[4] = 0;
+  if (tid == 0) L.misc[4] = L.misc[6] = 0;
   __syncthreads();
 
   // --- rest of collide's awake gating (contact_manager.py:191-197), in order ---
@@ -873,7 +878,6 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
     uint16_t* clb = cla + kGateChunk;
     uint16_t* cfl = clb + kGateChunk;  // bit 0 evaluated this step, bit 1 touching changed
     int* wcount = L.scan;
-    const int lane = tid & 63, wv = tid >> 6;
     for (int chunk = 0; chunk < used; chunk += kGateChunk) {
       const int cend = min(used, chunk + kGateChunk);
       for (int base = chunk; base < cend; base += kBlock) {
@@ -968,9 +972,22 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   const int j0 = d.w_joint_off ? d.w_joint_off[w] : 0;
   const int nj = d.w_joint_off ? d.w_joint_off[w + 1] - j0 : 0;
   for (int k = tid; k < nj; k += kBlock) d.j_flag[j0 + k] = 0;
+  // f(body, k) for the k-th body of more than kHubContacts contacts, by every wavefront
+  auto for_hubs = [&](auto&& f) {
+    int h = 0;
+    for (int base = 0; base < nb; base += 64) {
+      const int i = base + lane;
+      unsigned long long m = __ballot(i < nb && !(L.bst[i] & 1) && L.off[i + 1] - L.off[i] > kHubContacts);
+      for (; m; m &= m - 1) f(base + __ffsll(m) - 1, h++);
+    }
+  };
   for (int i = tid; i < nb; i += kBlock) {  // restore ascending slot order per body
     if (L.bst[i] & 1) continue;  // (static bodies' contacts are not walked: the ground's are many)
     int beg = L.off[i], end = L.off[i + 1];
+    if (end - beg > kHubContacts) {
+      L.misc[6] = 1;
+      continue;
+    }
     for (int k = beg + 1; k < end; ++k) {
       const uint32_t e = L.adj[k];
       int j = k - 1;
@@ -981,11 +998,42 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
       L.adj[j + 1] = e;
     }
     bool twice = false;
-    for (int k = beg + 1; k < end; ++k)
-      for (int j = beg; j < k; ++j) twice |= (L.adj[j] >> 16) == (L.adj[k] >> 16);
+    for (int k = beg + 1; k < end; ++k) {
+      const uint32_t o = L.adj[k] >> 16;
+#pragma unroll 4
+      for (int j = beg; j < k; ++j) twice |= (L.adj[j] >> 16) == o;
+    }
     if (twice) L.bst[i] |= 64;
   }
   __syncthreads();
+  const bool hubs = L.misc[6] != 0;
+  if (hubs) {  // through the entries' places in i_rank, which is free here and holds two a contact
+    uint32_t* sorted = (uint32_t*)(d.i_rank + cb);
+    for_hubs([&](int b, int h) {
+      const int beg = L.off[b], end = L.off[b + 1];
+      for (int k0 = beg + 64 * ((wv + h) % (kBlock / 64)); k0 < end; k0 += kBlock) {
+        const int k = k0 + lane;
+        const uint32_t e = L.adj[k < end ? k : beg];
+        int rank = 0;
+        bool twice = false;
+#pragma unroll 8
+        for (int j = beg; j < end; ++j) {
+          const uint32_t x = L.adj[j];
+          rank += (x & 0xFFFFu) < (e & 0xFFFFu);
+          twice |= (x >> 16 == e >> 16) & (j != k);
+        }
+        if (k < end) {
+          sorted[beg + rank] = e;
+          if (twice) L.bst[b] |= 64;  // (all that write it set the same bit)
+        }
+      }
+    });
+    __syncthreads();
+    for_hubs([&](int b, int) {
+      for (int k = L.off[b] + tid; k < L.off[b + 1]; k += kBlock) L.adj[k] = sorted[k];
+    });
+    __syncthreads();
+  }
 
   // --- depth-first island search (world.py:494-580), one wavefront ---
   // The walk itself only has to find the order in which bodies are taken off the stack.  A body's
@@ -999,7 +1047,6 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   int* isl_c = d.i_contacts + cb;
   int4* info = d.i_info + b0;
   if (tid < 64) {
-    const int lane = tid;
     int nbi_tot = 0, nisl = 0, njt = 0;
     for (int base = 0; base < nb; base += 64) {
       unsigned long long ahead = ~0ull;  // bodies of this 64 that are still to be looked at
@@ -1134,43 +1181,73 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   const int nisl = L.misc[0], nbi_tot = L.misc[1], qbase = L.misc[3];
   // A body takes, in adjacency order, its contacts with static bodies and with bodies that come
   // after it; the others were taken before.  Places in the contact list follow by a prefix sum.
+  // A lane takes a body, a wavefront one of many contacts.
+  auto takes = [&](int p, int k) {
+    const int o = (int)(L.adj[k] >> 16);
+    return (bool)((L.bst[o] & 1) | (L.bidx[o] > p));
+  };
   for (int b = tid; b < nb; b += kBlock) {
-    if ((L.bst[b] & (1 | 16)) != 16) continue;
+    if ((L.bst[b] & (1 | 16)) != 16 || L.off[b + 1] - L.off[b] > kHubContacts) continue;
     const int p = L.bidx[b];
     int n = 0;
-    for (int k = L.off[b]; k < L.off[b + 1]; ++k) {
-      const int o = (int)(L.adj[k] >> 16);
-      n += (L.bst[o] & 1) || L.bidx[o] > p;
-    }
+    for (int k = L.off[b]; k < L.off[b + 1]; ++k) n += takes(p, k);
     L.cur[p] = n;
   }
+  if (hubs)
+    for_hubs([&](int b, int h) {
+      if (h % (kBlock / 64) != wv || !(L.bst[b] & 16)) return;
+      const int p = L.bidx[b], end = L.off[b + 1];
+      int n = 0;
+      for (int k0 = L.off[b]; k0 < end; k0 += 64) n += __popcll(__ballot(k0 + lane < end && takes(p, k0 + lane)));
+      if (lane == 0) L.cur[p] = n;
+    });
   __syncthreads();
   const int nci_tot = block_exclusive_scan<B>(L.cur, nbi_tot, L.scan);
+  auto place = [&](int b, int p, int k, int c, uint32_t rank_b) {  // entry k of body b as contact c of the list
+    const int sl = (int)(L.adj[k] & 0xFFFFu), o = (int)(L.adj[k] >> 16);
+    const bool o_static = (L.bst[o] & 1) != 0;
+    // the contact's rank in the other body's sequence: that body's contacts taken before it
+    uint32_t rank_o = 0;
+    if (!o_static) {
+#pragma unroll 4
+      for (int q = L.off[o]; q < L.off[o + 1]; ++q) {
+        const uint32_t e = L.adj[q];
+        const int x = (int)(e >> 16);
+        rank_o += !(L.bst[x] & 1) & ((L.bidx[x] < p) | ((x == b) & ((int)(e & 0xFFFFu) < sl)));
+      }
+    }
+    isl_c[c] = sl;
+    d.i_rank[cb + c] = make_uint2((uint32_t)b, rank_b | rank_o << 16);
+    d.i_order[cb + c] = o_static ? 0xFFFFu : (uint32_t)o;
+  };
   for (int b = tid; b < nb; b += kBlock) {
     if ((L.bst[b] & (1 | 16)) != 16) continue;
     const int p = L.bidx[b], first = L.cur[p], beg = L.off[b], end = L.off[b + 1];
     L.slist[p] = (uint16_t)first;
+    if (end - beg > kHubContacts) continue;
     const int before = end - beg - ((p + 1 < nbi_tot ? L.cur[p + 1] : nci_tot) - first);
     int j = 0;
-    for (int k = beg; k < end; ++k) {
-      const int sl = (int)(L.adj[k] & 0xFFFFu), o = (int)(L.adj[k] >> 16);
-      const bool o_static = (L.bst[o] & 1) != 0;
-      if (!o_static && L.bidx[o] < p) continue;
-      // the contact's rank in the other body's sequence: that body's contacts taken before it
-      uint32_t rank_o = 0;
-      if (!o_static)
-        for (int q = L.off[o]; q < L.off[o + 1]; ++q) {
-          const uint32_t e = L.adj[q];
-          const int x = (int)(e >> 16);
-          rank_o += !(L.bst[x] & 1) && (L.bidx[x] < p || (x == b && (int)(e & 0xFFFFu) < sl));
-        }
-      const int c = first + j;
-      isl_c[c] = sl;
-      d.i_rank[cb + c] = make_uint2((uint32_t)b, (uint32_t)(before + j) | rank_o << 16);
-      d.i_order[cb + c] = o_static ? 0xFFFFu : (uint32_t)o;
-      ++j;
-    }
+    for (int k = beg; k < end; ++k)
+      if (takes(p, k)) {
+        place(b, p, k, first + j, (uint32_t)(before + j));
+        ++j;
+      }
   }
+  if (hubs)
+    for_hubs([&](int b, int h) {
+      if (h % (kBlock / 64) != wv || !(L.bst[b] & 16)) return;
+      const int p = L.bidx[b], first = L.cur[p], beg = L.off[b], end = L.off[b + 1];
+      const int before = end - beg - ((p + 1 < nbi_tot ? L.cur[p + 1] : nci_tot) - first);
+      int n = 0;
+      for (int k0 = beg; k0 < end; k0 += 64) {
+        const int k = k0 + lane;
+        const bool mine = k < end && takes(p, k);
+        const unsigned long long m = __ballot(mine);
+        const int j = n + __popcll(m & ((1ull << lane) - 1));
+        if (mine) place(b, p, k, first + j, (uint32_t)(before + j));
+        n += __popcll(m);
+      }
+    });
   __syncthreads();
   // The contacts' dependency levels: one more than the latest level among their dynamic bodies'
   // contacts before them.  A lane polls its contacts in list order, which every dependency follows;

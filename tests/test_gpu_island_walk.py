@@ -24,12 +24,24 @@ def _ground():
     return _body("static", (0.0, 0.0), [_fix(("edge", (-90.0, 0.0), (90.0, 0.0)))])
 
 
-def crowded(n):
-    """A dynamic slab on the ground under n boxes: n + 1 contacts of one body."""
+def _boxes(n, y):
+    return [_body("dynamic", (1.1 * (k - 0.5 * (n - 1)), y), [_fix(("box", 0.5, 0.5), density=1.0, friction=0.5)])
+            for k in range(n)]
+
+
+def crowded(n, kind="dynamic"):
+    """A slab under n boxes: n contacts of one body and, on the ground, one more."""
+    slab = _body(kind, (0.0, 0.5), [_fix(("box", 0.6 * n, 0.5), density=2.0, friction=0.5)])
+    return _world([_ground(), slab] + _boxes(n, 1.49))
+
+
+def sandwich(n):
+    """n boxes between two dynamic slabs, the upper one of two fixtures side by side: contacts of two
+    crowded bodies, taken by the lower slab and by the boxes."""
     slab = _body("dynamic", (0.0, 0.5), [_fix(("box", 0.6 * n, 0.5), density=2.0, friction=0.5)])
-    boxes = [_body("dynamic", (1.1 * (k - 0.5 * (n - 1)), 1.49), [_fix(("box", 0.5, 0.5), density=1.0, friction=0.5)])
-             for k in range(n)]
-    return _world([_ground(), slab] + boxes)
+    lid = _body("dynamic", (0.0, 2.47), [_fix(_box(0.3 * n, 0.5, -0.3 * n), density=0.2, friction=0.5),
+                                         _fix(_box(0.3 * n, 0.5, 0.3 * n), density=0.2, friction=0.5)])
+    return _world([_ground(), slab] + _boxes(n, 1.49) + [lid])
 
 
 def doubled(n):
@@ -50,7 +62,9 @@ def singles(n):
                                  for k in range(n)])
 
 
-SCENES = {"crowded": [crowded(n) for n in (62, 63, 64, 65, 130)], "doubled": [doubled(n) for n in (1, 5, 28)],
+SCENES = {"crowded": [crowded(n) for n in (15, 16, 17, 62, 63, 64, 65, 130)],
+          "kinematic": [crowded(n, "kinematic") for n in (16, 17, 130, 300)],
+          "sandwich": [sandwich(n) for n in (7, 15, 16, 17, 130, 300)], "doubled": [doubled(n) for n in (1, 5, 28)],
           "singles": [singles(n) for n in (1, 62, 63, 64, 110)]}
 
 
@@ -81,3 +95,16 @@ def test_walk_agrees_with_the_large_worlds_search(prec, name):
     for path, st in out.items():
         for f in ("body_d", "body_i", "fix_d", "con_d", "con_i"):
             assert np.array_equal(getattr(st, f), getattr(ref, f)), (path, f)
+
+
+def test_a_crowded_body_costs_no_more_than_as_many_apart():
+    """The island search of 600 boxes on a slab against that of 600 on static ground (once 21 times it)."""
+    ms = {}
+    for kind in ("kinematic", "dynamic", "static"):
+        e = N.Engine("fp32")
+        e.upload(builder.scene_batch(crowded(600, kind)))
+        e.step_n(10, DT, 8, 3, graph=True)
+        ms[kind] = np.median([e.profile(1, DT, 8, 3)[N.STAGES.index("islands")] for _ in range(7)])
+        print(kind, ms[kind], flush=True)
+        e.close()
+    assert max(ms["kinematic"], ms["dynamic"]) < 3 * ms["static"]
