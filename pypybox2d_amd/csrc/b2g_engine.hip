@@ -91,12 +91,12 @@ constexpr int kBigPairsBlock = 1024;  // k_pairs workgroup for the largest world
 constexpr int kMaxLds = 163840;  // LDS per workgroup on gfx950
 constexpr int kProfileBatch = 128;  // steps per event read-back in b2g_profile_step
 constexpr int kSizeClasses = 16;
-// q_cls layout: [0, 16) island count per class, [16, 32) cursors,
-// [32] islands in team classes, [33] wavefronts for them,
-// [34, 50) first wavefront per class, [50, 66) first queue entry per class,
-// [66, 82) first workgroup of k_solve_group per class, [82] its workgroups for groups,
-// [83] the lowest class solved by groups (kSizeClasses: k_solve takes every island)
-constexpr int kQHeavy = 2 * kSizeClasses, kQHeavyWaves = kQHeavy + 1, kQWaveBase = kQHeavy + 2,
+// q_cls layout, rows of a value per class: islands by queue_class and by group_class, cursors; islands in
+// team classes and wavefronts for them; islands, first wavefront and first queue entry per class as
+// k_order_islands has queued them; first workgroup of k_solve_group per class, its workgroups for groups and
+// the lowest class solved by groups (kSizeClasses: k_solve takes every island)
+constexpr int kQByGroup = kSizeClasses, kQCursor = 2 * kSizeClasses, kQHeavy = 3 * kSizeClasses,
+              kQHeavyWaves = kQHeavy + 1, kQCount = kQHeavy + 2, kQWaveBase = kQCount + kSizeClasses,
               kQBase = kQWaveBase + kSizeClasses, kQGroupBase = kQBase + kSizeClasses,
               kQGroupBlocks = kQGroupBase + kSizeClasses, kQGroupLow = kQGroupBlocks + 1, kQcls = kQGroupLow + 1;
 
@@ -128,9 +128,7 @@ inline bool groups_allowed(int vel_iters) { return (vel_iters + 1ll) * kGroupMax
 __host__ __device__ inline int group_waves(int cls) {
   return cls <= 5 ? 1 : (cls >= 8 ? kGroupWaves : 1 << (cls - 5));
 }
-// Is cls a class whose islands of up to kGroupMaxContacts get two contacts a lane?  The top class
-// holds islands of any size whose state did not fit a team's share (queue_class).
-__host__ __device__ inline bool group_two(int cls) { return cls == kGroupTopClass || cls == kSizeClasses - 1; }
+__host__ __device__ inline bool group_two(int cls) { return cls == kGroupTopClass; }  // two contacts a lane
 constexpr int kIslandTimeFields = 6;  // int64 per island of b2g_island_times
 
 // Team size of a heavy size class: 64 lanes from full_cls up, halved per class
@@ -166,6 +164,13 @@ __device__ __forceinline__ int queue_class(const D& d, int nc, int nbi) {
     if (ts < kSolveBlock && team_lds_bytes(nbi) > d.team_lds / (kSolveBlock / ts)) c = kSizeClasses - 1;
   }
   return c;
+}
+
+// The same where groups solve the islands of up to kGroupMaxContacts: those have room for any number
+// of bodies that as many contacts hold together, so that a team's share of LDS does not matter to them.
+template <typename D>
+__device__ __forceinline__ int group_class(const D& d, int nc, int nbi) {
+  return nc <= kGroupMaxContacts ? size_class(nc) : queue_class(d, nc, nbi);
 }
 
 // The sweep period of an island whose contacts have one-sweep dependency levels 1..depth and
@@ -794,7 +799,7 @@ __host__ __device__ inline size_t island_smem_bytes(int nb, int nf, int ccap) {
   // free: a bit per contact slot, so that the same worlds fit whose joints the other path refuses
   s += ((size_t)(ccap + 31) / 32 * 4 + 15) & ~(size_t)15;
   s += (size_t)kBlock * 4;
-  s += 64 * 4;  // misc: 16 scalars, 16 class counts, spare
+  s += 64 * 4;  // misc: 16 scalars, 32 class counts, spare
   return s;
 }
 
@@ -1327,17 +1332,18 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
     }
     d.i_jidx[j0 + k] = make_int4(idx[0], idx[1], idx[2], idx[3]);
   }
-  int* ccount = L.misc + 16;  // islands per size class, then one global add per class
-  if (tid < kSizeClasses) ccount[tid] = 0;
+  int* ccount = L.misc + 16;  // islands per class of either kind, then one global add per class
+  if (tid < 2 * kSizeClasses) ccount[tid] = 0;
   __syncthreads();
   for (int k = tid; k < nisl; k += kBlock) {
     int4 in = info[k];
     d.q_isl[qbase + k] = make_int4(w, b0 + in.x, in.y, cb + in.z);
     d.q_nc[qbase + k] = in.w;
     atomicAdd(&ccount[queue_class(d, in.w & 0x3FFFFFFF, in.y & 0xFFFF)], 1);
+    atomicAdd(&ccount[kQByGroup + group_class(d, in.w & 0x3FFFFFFF, in.y & 0xFFFF)], 1);
   }
   __syncthreads();
-  if (tid < kSizeClasses && ccount[tid] > 0) atomicAdd(&d.q_cls[tid], ccount[tid]);
+  if (tid < 2 * kSizeClasses && ccount[tid] > 0) atomicAdd(&d.q_cls[tid], ccount[tid]);
   for (int k = tid; k < nci_tot; k += kBlock) {
     const int s = isl_c[k];
     int2 pr = d.c_pair[cb + s];
@@ -2799,7 +2805,7 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
       const int per = kSolveBlock / TS;
       const int team = l / TS, t = l % TS;
       const int q = d.q_cls[kQBase + cls] + (g - d.q_cls[kQWaveBase + cls]) * per + team;
-      const int qend = d.q_cls[kQBase + cls] + d.q_cls[cls];
+      const int qend = d.q_cls[kQBase + cls] + d.q_cls[kQCount + cls];
       if (q < qend) {
         const int4 in = d.qs_isl[q];
         const int nbi = in.z & 0xFFFF, period = (int)((uint32_t)in.z >> 16);
@@ -2809,8 +2815,8 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
         const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
         const bool fits = team_lds_bytes(nbi) <= share;
         SolveMarks mk{0, 0};
-        if (island_has_joints(d, in.x, in.y) || (grouped && nci <= kGroupMaxContacts)) {
-          // k_solve_joints or k_solve_group takes it
+        if (island_has_joints(d, in.x, in.y)) {
+          // k_solve_joints takes it
         } else if (fits) {
           solve_island_team(d, in.x, in.y, nbi, in.w, nci, last_allow, period, team_lds + team * share, t, TS, mk);
           if (d.i_time && t == 0) record_island_time(d, q, t0, nci, nbi, TS, period, mk);
@@ -3092,12 +3098,12 @@ __device__ __forceinline__ void solve_group_block(const Dev<T>& d, int cls, int 
   const int waves = J == 2 ? kGroupWaves : group_waves(cls), per = kGroupWaves / waves;
   const int team = (threadIdx.x >> 6) / waves, t = threadIdx.x - team * waves * 64;
   const int q = d.q_cls[kQBase + cls] + (g - d.q_cls[kQGroupBase + cls]) * per + team;
-  if (q >= d.q_cls[kQBase + cls] + d.q_cls[cls]) return;
+  if (q >= d.q_cls[kQBase + cls] + d.q_cls[kQCount + cls]) return;
   const int4 in = d.qs_isl[q];
   const int nc = d.qs_nc[q];
   const int nbi = in.z & 0xFFFF, nci = nc & 0x3FFFFFFF, last_allow = (nc >> 30) & 1;
-  // islands with joints are left to k_solve_joints, larger ones of the top class to k_solve
-  if (nci > kGroupMaxContacts || island_has_joints(d, in.x, in.y)) return;
+  // (what the LDS holds; group_class sees to it)
+  if (nci > kGroupMaxContacts || island_has_joints(d, in.x, in.y)) return;  // k_solve_joints takes it
   const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
   SolveMarks mk{0, 0};
   solve_island_group<T, J>(d, in.x, in.y, nbi, in.w, nci, last_allow, st + team * (waves * 64 * J + 1), &bar[team],
@@ -3118,13 +3124,12 @@ __global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_e
   const int low = d.q_cls[kQGroupLow];
   if (low >= kSizeClasses) return;  // k_solve takes every island
   const int groups = d.q_cls[kQGroupBlocks];
-  const int n = *d.q_count, light = d.q_cls[kQBase + low] + d.q_cls[low];
+  const int n = *d.q_count, light = d.q_cls[kQBase + low] + d.q_cls[kQCount + low];
   const int blocks = groups + (n - light + kGroupBlock - 1) / kGroupBlock;
   for (int g = blockIdx.x; g < blocks; g += gridDim.x) {
     if (g < groups) {
       int cls = low;  // the classes own consecutive workgroup ranges, highest class first
-      while (cls < kGroupTopClass && g < d.q_cls[kQGroupBase + cls]) ++cls;
-      if (g < d.q_cls[kQGroupBase + cls]) cls = kSizeClasses - 1;
+      while (g < d.q_cls[kQGroupBase + cls]) ++cls;  // (the highest class's range begins at 0)
       if (threadIdx.x < kGroupWaves) bar[threadIdx.x] = 0;
       __syncthreads();
       if (group_two(cls)) solve_group_block<T, 2>(d, cls, g, st, bar, red);
@@ -4196,7 +4201,7 @@ __global__ void __launch_bounds__(kBigBlock) k_islands_big(Dev<T> d, int sort_ca
   __syncthreads();
   // --- queue, island-local contact ends, ranks oriented as (body A, body B) ---
   if (tid == 0) sh[2] = nisl > 0 ? atomicAdd(d.q_count, nisl) : 0;
-  if (tid < kSizeClasses) scan[tid] = 0;
+  if (tid < 2 * kSizeClasses) scan[tid] = 0;
   __syncthreads();
   const int qbase = sh[2];
   for (int k = tid; k < nisl; k += kBigBlock) {
@@ -4204,9 +4209,10 @@ __global__ void __launch_bounds__(kBigBlock) k_islands_big(Dev<T> d, int sort_ca
     d.q_isl[qbase + k] = make_int4(w, b0 + in.x, in.y, cb + in.z);
     d.q_nc[qbase + k] = in.w;
     atomicAdd(&scan[queue_class(d, in.w & 0x3FFFFFFF, in.y & 0xFFFF)], 1);
+    atomicAdd(&scan[kQByGroup + group_class(d, in.w & 0x3FFFFFFF, in.y & 0xFFFF)], 1);
   }
   __syncthreads();
-  if (tid < kSizeClasses && scan[tid] > 0) atomicAdd(&d.q_cls[tid], scan[tid]);
+  if (tid < 2 * kSizeClasses && scan[tid] > 0) atomicAdd(&d.q_cls[tid], scan[tid]);
   if (tid == 0) {
     d.w_nisl[w] = nisl;
     d.w_itot[w] = make_int2(nbi_tot, nci_tot);
@@ -5432,7 +5438,7 @@ __global__ void k_reset_queue(Dev<T> d) {
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) *d.q_count = 0;
     if (threadIdx.x == 0 && d.ev_count) *d.ev_count = 0;  // events are those of the last step
-    if (threadIdx.x < kQWaveBase) d.q_cls[threadIdx.x] = 0;
+    if (threadIdx.x < kQCount) d.q_cls[threadIdx.x] = 0;
   }
 }
 
@@ -5495,43 +5501,54 @@ __global__ void k_disable(Dev<T> d, const int* ws, int n) {
 // 256 worlds 2.60 / 3.26, 509 2.58 / 3.34, 700 (load about 630) 3.03 / 3.55, 1000 (about 900)
 // 4.07 / 3.65; 3001 long-tailed worlds (about 520) 2.90 / 3.41.  Every class from 5 up has to fit
 // (k_solve has teams for them); smaller islands get a wavefront each while there is room, else a lane.
+struct GroupPlan {
+  int low, blocks, base[kGroupTopClass + 1];
+};
 template <typename T>
-__device__ void plan_groups(const Dev<T>& d) {
-  int blocks = 0, load = 0, low = kSizeClasses;
+__device__ void plan_groups(const Dev<T>& d, const int* count, GroupPlan& p) {  // count: islands by group_class
+  int load = 0;
+  p.blocks = 0;
+  p.low = kSizeClasses;
   if (d.group_load > 0 && d.heavy_class <= kGroupTopClass) {
-    for (int c = kSizeClasses - 1; c > 0; c = c == kSizeClasses - 1 ? kGroupTopClass : c - 1) {
-      const int n = d.q_cls[c];
-      const int need = group_two(c) ? n : (n * group_waves(c) + kGroupWaves - 1) / kGroupWaves;
+    for (int c = kGroupTopClass; c > 0; --c) {
+      const int n = count[c];
+      const int need = (n * group_waves(c) + kGroupWaves - 1) / kGroupWaves;
       load += need * (group_two(c) ? 16 : (c > 5 ? 1 << (c - 5) : 1));
       if (load > 8 * d.group_load) break;
-      d.q_cls[kQGroupBase + c] = blocks;
-      blocks += need;
-      low = c;
+      p.base[c] = p.blocks;
+      p.blocks += need;
+      p.low = c;
     }
-    if (low > kGroupLastClass) low = kSizeClasses;
+    if (p.low > kGroupLastClass) p.low = kSizeClasses;
   }
-  d.q_cls[kQGroupBlocks] = blocks;
-  d.q_cls[kQGroupLow] = low;
 }
 
-// Orders the island queue by size class, largest first, so that the lanes of
+// Orders the island queue by class, largest first, so that the lanes of
 // a wave of k_solve carry islands of similar length.  Each block takes a
 // contiguous chunk of the queue, counts its classes in LDS and reserves its
-// ranges with one global atomic per class.
+// ranges with one global atomic per class.  The classes are group_class's
+// where groups are chosen (each block finds the plan), else queue_class's.
 template <typename T>
 __global__ void k_order_islands(Dev<T> d) {
-  __shared__ int base[kSizeClasses], lcnt[kSizeClasses], lbase[kSizeClasses];
+  __shared__ int count[2 * kSizeClasses], base[kSizeClasses], lcnt[kSizeClasses], lbase[kSizeClasses];
+  __shared__ GroupPlan plan;
+  if (threadIdx.x < 2 * kSizeClasses) count[threadIdx.x] = d.q_cls[threadIdx.x];
   if (threadIdx.x < kSizeClasses) lcnt[threadIdx.x] = 0;
+  __syncthreads();
   if (threadIdx.x == 0) {
+    plan_groups(d, count + kQByGroup, plan);
+    const int* cnt = plan.low < kSizeClasses ? count + kQByGroup : count;
     int run = 0, waves = 0;
     for (int c = kSizeClasses - 1; c >= 0; --c) {
       base[c] = run;
-      const int nc = d.q_cls[c];
+      const int nc = cnt[c];
       if (blockIdx.x == 0) {
+        d.q_cls[kQCount + c] = nc;
         d.q_cls[kQBase + c] = run;
         d.q_cls[kQWaveBase + c] = waves;
         if (c >= d.heavy_class)
           waves += (nc * team_size(c, d.team_full_class, d.team_max) + kSolveBlock - 1) / kSolveBlock;
+        if (c >= plan.low && c <= kGroupTopClass) d.q_cls[kQGroupBase + c] = plan.base[c];
       }
       run += nc;
       if (c == d.heavy_class && blockIdx.x == 0) {
@@ -5539,25 +5556,30 @@ __global__ void k_order_islands(Dev<T> d) {
         d.q_cls[kQHeavyWaves] = waves;
       }
     }
-    if (blockIdx.x == 0) plan_groups(d);
+    if (blockIdx.x == 0) {
+      d.q_cls[kQGroupBlocks] = plan.blocks;
+      d.q_cls[kQGroupLow] = plan.low;
+    }
   }
   __syncthreads();
+  const bool grouped = plan.low < kSizeClasses;
+  auto class_of = [&](int nc, int nbi) { return grouped ? group_class(d, nc, nbi) : queue_class(d, nc, nbi); };
   const int n = *d.q_count;
   const int per = (n + gridDim.x - 1) / gridDim.x;
   const int q0 = blockIdx.x * per, q1 = min(n, q0 + per);
   for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x)
-    atomicAdd(&lcnt[queue_class(d, d.q_nc[q] & 0x3FFFFFFF, d.q_isl[q].z & 0xFFFF)], 1);
+    atomicAdd(&lcnt[class_of(d.q_nc[q] & 0x3FFFFFFF, d.q_isl[q].z & 0xFFFF)], 1);
   __syncthreads();
   if (threadIdx.x < kSizeClasses) {
     const int c = threadIdx.x;
-    lbase[c] = lcnt[c] > 0 ? base[c] + atomicAdd(&d.q_cls[kSizeClasses + c], lcnt[c]) : 0;
+    lbase[c] = lcnt[c] > 0 ? base[c] + atomicAdd(&d.q_cls[kQCursor + c], lcnt[c]) : 0;
     lcnt[c] = 0;
   }
   __syncthreads();
   for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
     const int nc = d.q_nc[q];
     const int4 isl = d.q_isl[q];
-    const int c = queue_class(d, nc & 0x3FFFFFFF, isl.z & 0xFFFF);
+    const int c = class_of(nc & 0x3FFFFFFF, isl.z & 0xFFFF);
     const int pos = lbase[c] + atomicAdd(&lcnt[c], 1);
     d.qs_isl[pos] = isl;
     d.qs_nc[pos] = nc;
@@ -5578,7 +5600,7 @@ __global__ void __launch_bounds__(kPrefixBlock) k_order_team_islands(Dev<T> d) {
   __shared__ int bins[kTeamSortBins], scan[kPrefixBlock];
   const int c = blockIdx.x;
   if (c < d.heavy_class && c < d.q_cls[kQGroupLow]) return;
-  const int b = d.q_cls[kQBase + c], n = d.q_cls[c];
+  const int b = d.q_cls[kQBase + c], n = d.q_cls[kQCount + c];
   if (n < 2) return;
   const int TS = c >= d.q_cls[kQGroupLow] ? 2 * kGroupBlock : team_size(c, d.team_full_class, d.team_max);
   auto bin_of = [&](const int4& in, int nc) {

@@ -93,3 +93,32 @@ def test_many_iterations_on_a_body_of_many_contacts(prec, iters):
     assert gt[2] >= 300 and gt[4] == (64 if iters <= 4103 else 32) and tt[4] == 32
     for f in ("body_d", "con_d", "con_i"):
         assert np.array_equal(getattr(groups, f), getattr(teams, f)), f
+
+
+def _towers(heights):
+    bodies = [_body("static", (0.0, 0.0), [_fix(("edge", (-90.0, 0.0), (90.0, 0.0)))])]
+    bodies += [_body("dynamic", (2.0 * (k - 0.5 * len(heights)), 0.49 + 0.99 * r), [_fix(("box", 0.5, 0.5), density=1.0)])
+               for k, h in enumerate(heights) for r in range(h)]
+    return {"gravity": (0.0, -10.0), "bodies": bodies, "do_sleep": False, "warm_starting": True}
+
+
+@pytest.mark.parametrize("team_lds", [16384, 24576, 32768])
+def test_groups_do_not_depend_on_the_teams_memory(team_lds):
+    """Towers of 115 boxes do not fit a team's share of LDS in most of its sizes; in groups they take two
+    wavefronts and their load all the same (3 workgroups, of which those of 40 boxes need one)."""
+    batch = builder.scene_batch(_towers([115] * 8 + [40] * 8))
+    out = []
+    for load in (3, 0):
+        e = N.Engine("fp64")
+        e.set_param("group_load", load)
+        e.set_param("team_lds", team_lds)
+        e.set_param("island_times", 1)
+        e.upload(batch)
+        e.step_n(4, DT, 8, 3, graph=True)
+        out.append((e.download(), e.island_times()))
+        print(team_lds, load, "done", flush=True)
+        e.close()
+    assert sorted(set(out[0][1][:, 2].tolist())) == [40, 115] and set(out[0][1][:, 4].tolist()) == {64}
+    assert 8 in out[1][1][:, 4]
+    for f in ("body_d", "con_d", "con_i"):
+        assert np.array_equal(getattr(out[0][0], f), getattr(out[1][0], f)), f
