@@ -120,6 +120,8 @@ constexpr int kGroupPolls = 1 << 26;
 constexpr int kSolvePolls = 16;
 constexpr int kGroupTopClass = 9;     // the largest islands with a lane per two contacts
 constexpr int kGroupLastClass = 5;     // groups take every island of this class and above, or none
+constexpr int kGroupMinClass = 2;      // ... and of no class below this one
+constexpr int kGroupSmallBlocks = kCus; // most workgroups for the classes between (twice as many without the least)
 constexpr int kGroupMaxContacts = (1 << (kGroupTopClass + 1)) - 2;
 // May islands be solved by groups in a step of these iterations (up to 4103)?
 inline bool groups_allowed(int vel_iters) { return (vel_iters + 1ll) * kGroupMaxContacts * kSolvePolls <= kGroupPolls; }
@@ -249,6 +251,7 @@ struct Dev {
   int team_lds;         // LDS bytes per wavefront of teams
   int team_max;         // largest team below the top class (8, 16, 32 or 64)
   int group_load;       // most load of k_solve_group (plan_groups); 0: none
+  bool group_only;      // k_solve_group takes every island, k_solve is not launched
   // worlds
   const int* w_body_off;
   const int* w_fix_off;
@@ -3125,7 +3128,9 @@ __global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_e
   if (low >= kSizeClasses) return;  // k_solve takes every island
   const int groups = d.q_cls[kQGroupBlocks];
   const int n = *d.q_count, light = d.q_cls[kQBase + low] + d.q_cls[kQCount + low];
-  const int blocks = groups + (n - light + kGroupBlock - 1) / kGroupBlock;
+  // islands beyond the groups: a lane each, in as few lanes of a workgroup as give every compute unit some
+  const int waves = (n - light + 64 * kCus - 1) / (64 * kCus), lanes = 64 * min(max(waves, 1), kGroupWaves);
+  const int blocks = groups + (n - light + lanes - 1) / lanes;
   for (int g = blockIdx.x; g < blocks; g += gridDim.x) {
     if (g < groups) {
       int cls = low;  // the classes own consecutive workgroup ranges, highest class first
@@ -3136,8 +3141,8 @@ __global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_e
       else solve_group_block<T, 1>(d, cls, g, st, bar, red);
       __syncthreads();  // the next islands reuse the LDS
     } else {
-      const int q = light + (g - groups) * kGroupBlock + (int)threadIdx.x;
-      if (q < n) {
+      const int q = light + (g - groups) * lanes + (int)threadIdx.x;
+      if ((int)threadIdx.x < lanes && q < n) {
         const long long t0 = d.i_time ? (long long)wall_clock64() : 0;
         const int4 in = d.qs_isl[q];
         const int nc = d.qs_nc[q];
@@ -5500,7 +5505,12 @@ __global__ void k_disable(Dev<T> d, const int* ws, int n) {
 // workgroup of class 8.  Solve stage in ms with and without groups, mixed worlds of 32 to 512 bodies:
 // 256 worlds 2.60 / 3.26, 509 2.58 / 3.34, 700 (load about 630) 3.03 / 3.55, 1000 (about 900)
 // 4.07 / 3.65; 3001 long-tailed worlds (about 520) 2.90 / 3.41.  Every class from 5 up has to fit
-// (k_solve has teams for them); smaller islands get a wavefront each while there is room, else a lane.
+// (k_solve has teams for them).  Smaller islands get a wavefront each while each compute unit has at most
+// two workgroups of those of 7 contacts and more, one of those of 3 and more, else a lane.  Towers of 3, 5, 10
+// and 15 boxes, solve in us by wavefronts / lanes: about 250 workgroups - / -, 62 / 95, 115 / 200, 142 / 290;
+// 500 of them 105 / 83, 95 / 99, 186 / 204, 240 / 311; 1250 to 2500 - / -, 354 / 157, 408 / 250, 641 / 395.
+// Islands of one or two contacts (a box on the ground) end as soon in a lane: a wavefront each took 142 us
+// for 12000 of them, where lanes take 65.
 struct GroupPlan {
   int low, blocks, base[kGroupTopClass + 1];
 };
@@ -5509,18 +5519,17 @@ __device__ void plan_groups(const Dev<T>& d, const int* count, GroupPlan& p) {  
   int load = 0;
   p.blocks = 0;
   p.low = kSizeClasses;
-  if (d.group_load > 0 && d.heavy_class <= kGroupTopClass) {
-    for (int c = kGroupTopClass; c > 0; --c) {
-      const int n = count[c];
-      const int need = (n * group_waves(c) + kGroupWaves - 1) / kGroupWaves;
-      load += need * (group_two(c) ? 16 : (c > 5 ? 1 << (c - 5) : 1));
-      if (load > 8 * d.group_load) break;
-      p.base[c] = p.blocks;
-      p.blocks += need;
-      p.low = c;
-    }
-    if (p.low > kGroupLastClass) p.low = kSizeClasses;
+  if (d.group_load == 0 || d.heavy_class > kGroupTopClass) return;
+  int small = 0;
+  for (int c = kGroupTopClass; c >= kGroupMinClass; --c) {
+    const int need = (count[c] * group_waves(c) + kGroupWaves - 1) / kGroupWaves;
+    if (c < kGroupLastClass && (small += need) > (c > kGroupMinClass ? 2 : 1) * kGroupSmallBlocks) break;
+    if (c >= kGroupLastClass) load += need * (group_two(c) ? 16 : 1 << (c - kGroupLastClass));
+    p.base[c] = p.blocks;
+    p.blocks += need;
+    p.low = c;
   }
+  if (!d.group_only && (load > 8 * d.group_load || p.blocks == 0)) p.low = kSizeClasses;
 }
 
 // Orders the island queue by class, largest first, so that the lanes of
@@ -5599,10 +5608,11 @@ template <typename T>
 __global__ void __launch_bounds__(kPrefixBlock) k_order_team_islands(Dev<T> d) {
   __shared__ int bins[kTeamSortBins], scan[kPrefixBlock];
   const int c = blockIdx.x;
-  if (c < d.heavy_class && c < d.q_cls[kQGroupLow]) return;
+  const bool grouped = d.q_cls[kQGroupLow] < kSizeClasses;
+  if (c < (grouped ? kGroupLastClass : d.heavy_class)) return;  // (smaller ones: groups of all run at once)
   const int b = d.q_cls[kQBase + c], n = d.q_cls[kQCount + c];
   if (n < 2) return;
-  const int TS = c >= d.q_cls[kQGroupLow] ? 2 * kGroupBlock : team_size(c, d.team_full_class, d.team_max);
+  const int TS = grouped && c <= kGroupTopClass ? 2 * kGroupBlock : team_size(c, d.team_full_class, d.team_max);
   auto bin_of = [&](const int4& in, int nc) {
     const int est = team_island_length(in, nc, TS);
     return kTeamSortBins - 1 - (est < kTeamSortBins - 1 ? est : kTeamSortBins - 1);
@@ -6798,6 +6808,10 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
   d.pos_iters = pi;
   d.heavy_class = ctx->heavy_class;
   d.group_load = groups_allowed(vi) ? ctx->group_load : 0;
+  // Few enough contacts that the groups' load cannot reach its limit (8 eighths for 255 contacts, and rounding;
+  // plan_groups) and no island too large for them: k_solve would only be an empty launch.
+  d.group_only = d.group_load > 0 && ctx->heavy_class <= kGroupTopClass && ctx->max_ccap <= kGroupMaxContacts &&
+                 ctx->ncap / 31 + 8 <= 8 * d.group_load;
   d.team_full_class = ctx->team_full_class;
   d.team_lds = ctx->team_lds;
   d.team_max = ctx->team_max;
@@ -6901,7 +6915,8 @@ static int launch_step(b2g_ctx* ctx, double dt, int vi, int pi, bool first_pairs
       HIPCHK(hipEventRecord(ctx->fork_ev, st));
       HIPCHK(hipStreamWaitEvent(ctx->aux[0], ctx->fork_ev, 0));
     }
-    hipLaunchKernelGGL(k_solve<T>, dim3(swaves), dim3(kSolveBlock), ctx->team_lds, beside ? ctx->aux[0] : st, d);
+    if (!d.group_only)
+      hipLaunchKernelGGL(k_solve<T>, dim3(swaves), dim3(kSolveBlock), ctx->team_lds, beside ? ctx->aux[0] : st, d);
     if (d.group_load > 0) {
       const int ggrid = std::max(1, std::min(ctx->nb, 4096));
       hipLaunchKernelGGL(k_solve_group<T>, dim3(ggrid), dim3(kGroupBlock), 0, st, d);

@@ -122,3 +122,35 @@ def test_groups_do_not_depend_on_the_teams_memory(team_lds):
     assert 8 in out[1][1][:, 4]
     for f in ("body_d", "con_d", "con_i"):
         assert np.array_equal(getattr(out[0][0], f), getattr(out[1][0], f)), f
+
+
+def _step_ms(batch, load):
+    e = N.Engine("fp32")
+    e.set_param("group_load", load)
+    e.set_param("island_times", 1)
+    e.upload(batch)
+    e.step_n(4, DT, 8, 3, graph=True)
+    st, lanes = e.download(), e.island_times()[:, 4]
+    ms = min(float(e.profile(1, DT, 8, 3)[N.STAGES.index("solve")]) for _ in range(9))
+    e.close()
+    return st, lanes, ms
+
+
+@pytest.mark.parametrize("heights,copies,want", [([1] * 3, 1, 1), ([2] * 3, 700, 1), ([3] * 8, 1, 64), ([3] * 8, 256, 64),
+                                                 ([3] * 8, 257, 1), ([14] * 8, 513, 1), ([15] * 8, 512, 64),
+                                                 ([40, 3, 3, 1], 300, None), ([1] * 5, 3000, 1)])
+def test_small_islands_take_wavefronts_only_while_those_are_few(heights, copies, want):
+    """Towers of one class: of up to two contacts a lane each; of three and more a wavefront each while 256
+    workgroups of eight hold them, of seven and more while 512 do.  The group solver is no slower than the lanes and teams by more than
+    its launch costs."""
+    batch = L.concat([builder.scene_batch(_towers(heights))] * copies)
+    st, lanes, ms = _step_ms(batch, 768)
+    ref, _, ref_ms = _step_ms(batch, 0)
+    print(heights, copies, np.unique(lanes, return_counts=True), "%.3f ms, without groups %.3f" % (ms, ref_ms), flush=True)
+    if want is None:  # 40 high and 3 high in wavefronts, 1 high in a lane
+        assert np.count_nonzero(lanes == 64) == 3 * copies and np.count_nonzero(lanes == 1) == copies
+    else:
+        assert set(lanes.tolist()) == {want}
+    for f in ("body_d", "con_d", "con_i"):
+        assert np.array_equal(getattr(st, f), getattr(ref, f)), f
+    assert ms < 1.15 * ref_ms + 0.03
