@@ -806,31 +806,33 @@ __host__ __device__ inline size_t island_smem_bytes(int nb, int nf, int ccap) {
   return s;
 }
 
-// Exclusive scan of a[0..n) in place by one workgroup; returns the total.
+// Exclusive scan of a[0..n) in place by one workgroup; returns the total.  scratch: a value per wavefront.
 template <int B = kBlock>
 __device__ int block_exclusive_scan(int* a, int n, int* scratch) {
-  constexpr int kBlock = B;
-  const int tid = threadIdx.x;
-  const int per = (n + kBlock - 1) / kBlock;
-  const int beg = tid * per, end = min(n, beg + per);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int per = (n + B - 1) / B;
+  const int beg = min(n, tid * per), end = min(n, beg + per);
   int sum = 0;
   for (int i = beg; i < end; ++i) sum += a[i];
-  scratch[tid] = sum;
-  __syncthreads();
-  for (int off = 1; off < kBlock; off <<= 1) {
-    int v = tid >= off ? scratch[tid - off] : 0;
-    __syncthreads();
-    scratch[tid] += v;
-    __syncthreads();
+  int run = sum;  // up to and with this lane
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(run, off);
+    if (lane >= off) run += v;
   }
-  int run = scratch[tid] - sum;
+  if (lane == 63) scratch[wv] = run;
+  __syncthreads();
+  int total = 0;
+  run -= sum;
+  for (int k = 0; k < B / 64; ++k) {
+    const int v = scratch[k];
+    if (k < wv) run += v;
+    total += v;
+  }
   for (int i = beg; i < end; ++i) {
     int v = a[i];
     a[i] = run;
     run += v;
   }
-  __syncthreads();
-  int total = scratch[kBlock - 1];
   __syncthreads();
   return total;
 }
