@@ -174,6 +174,9 @@ B2G_API int b2g_last_error(b2g_ctx* ctx, char* buf, size_t n);
                           never with a heavy class above 9).  Results do not
                           depend on it. */
 #define B2G_PARAM_GROUP_LOAD 15
+/* B2G_PARAM_JOINT_LDS    (read only) bytes of LDS in which a wavefront each solves the
+                          uploaded batch's islands with joints; 0: a lane each. */
+#define B2G_PARAM_JOINT_LDS 16
 B2G_API int b2g_set_param(b2g_ctx* ctx, int32_t key, int32_t value);
 B2G_API int b2g_get_param(b2g_ctx* ctx, int32_t key, int32_t* value);
 

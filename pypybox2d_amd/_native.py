@@ -31,7 +31,7 @@ EXPORTS = ("b2g_version", "b2g_create", "b2g_destroy", "b2g_upload", "b2g_step",
 PARAMS = {"team_lds": 1, "heavy_class": 2, "solve_grid": 3, "team_full_class": 4, "large_worlds": 5,
           "island_times": 6, "solve_waves_per_cu": 7, "team_max": 8, "search_runs": 9, "pairs_wide": 10,
           "islands_wide": 11, "collide_block": 12, "tree_pairs": 13, "events": 14,
-          "group_load": 15}
+          "group_load": 15, "joint_lds": 16}
 
 # the stages b2g_profile_step times, in order
 STAGES = ("collide", "islands", "solve", "sync", "pairs")

@@ -109,6 +109,7 @@ __host__ __device__ inline int size_class(int nc) {  // floor(log2(nc + 1)), cap
 constexpr int kSolveBlock = 64;  // k_solve: one wavefront per workgroup
 constexpr int kJointLdsMax = 65536;   // most LDS of a joint island (k_solve_joints_lds)
 constexpr int kCus = 256;             // compute units
+constexpr int kJointWaves = 128;      // wavefronts of joint islands that run as fast as one (upload_batch)
 constexpr int kGroupBlock = 512;      // k_solve_group: eight wavefronts
 constexpr int kGroupWaves = kGroupBlock / 64;
 // Polls of a dataflow without its end: WERR_SCHEDULE.  At least one solve is always ready, and a poll in
@@ -3163,8 +3164,12 @@ __global__ void __launch_bounds__(kGroupBlock) __attribute__((amdgpu_waves_per_e
 // batches with joints.  Their bodies and contacts belong to no other island, so the order of the
 // two kernels does not matter.  k_solve_joints takes them a lane each, k_solve_joints_lds a
 // wavefront each where every world's joints and bodies fit its LDS.  Bound by the serial sweeps' reads: the testbed's bridge
-// (31 joints) takes 357 us a lane with its records in HBM and about 290 us in LDS.  Batches of more
-// worlds with joints than fit the chip's LDS side by side take the lanes, 64 islands a wavefront.
+// (31 joints) takes 357 us a lane with its records in HBM and about 290 us in LDS.  That lasts to about one
+// wavefront for each two compute units (the code of ten joint types is larger than the instruction
+// cache they share): bridges of 12 planks, solve in us by wavefronts / lanes, 64 worlds 193 / 212, 128 200 / 213, 192
+// 226 / 211, 512 298 / 215, 4000 1175 / 294.  Lanes pay for every joint type among the islands of a
+// wavefront (joint_lane_steps), wavefronts do not: 14 mechanisms a world, 128 worlds 187 / 237, 256 195 / 241, 320
+// 263 / 241, 1000 523 / 263.  So wavefronts take batches of up to 128 joints for each step of the lanes.
 template <typename T>
 __global__ void __launch_bounds__(64) k_solve_joints(Dev<T> d) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -6206,6 +6211,38 @@ static int ensure_event_buffers(b2g_ctx* ctx, Dev<T>& d) {
   return 0;
 }
 
+// The steps of a wavefront of k_solve_joints over a batch's joints, a lane for each set of joints that
+// share moving bodies: the k-th joints of all sets run together where they are of one type, else one
+// type after another.
+static int joint_lane_steps(const b2g_batch* b) {
+  std::vector<uint16_t> types;  // at k: the types among the k-th joints of the sets
+  for (int w = 0; w < b->n_worlds; ++w) {
+    const int b0 = b->body_off[w], wnb = b->body_off[w + 1] - b0;
+    std::vector<int> parent(wnb), joints(wnb, 0);
+    for (int i = 0; i < wnb; ++i) parent[i] = i;
+    auto find = [&](int i) {
+      while (parent[i] != i) i = parent[i] = parent[parent[i]];
+      return i;
+    };
+    auto moves = [&](int i) { return i >= 0 && b->body_i[(size_t)(b0 + i) * B2G_BODY_NI + B2G_BI_TYPE] != BT_STATIC; };
+    for (int pass = 0; pass < 2; ++pass)
+      for (int j = b->joint_off[w]; j < b->joint_off[w + 1]; ++j) {
+        const int32_t* ji = b->joint_i + (size_t)j * B2G_JOINT_NI;
+        const int ba = ji[B2G_JI_BODY_A], bb = ji[B2G_JI_BODY_B];
+        if (pass == 0) {
+          if (moves(ba) && moves(bb)) parent[find(ba)] = find(bb);
+        } else if (moves(ba) || moves(bb)) {
+          const size_t k = (size_t)joints[find(moves(ba) ? ba : bb)]++;
+          if (types.size() <= k) types.resize(k + 1, 0);
+          types[k] |= (uint16_t)(1u << ji[B2G_JI_TYPE]);
+        }
+      }
+  }
+  int steps = 0;
+  for (uint16_t t : types) steps += __builtin_popcount(t);
+  return steps;
+}
+
 template <typename T>
 static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
   const int nw = b->n_worlds;
@@ -6655,16 +6692,12 @@ static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
     d.w_jnc_off = wjn;
     d.jnc = jncd;
     ctx->nj = nj;
-    int joint_worlds = 0;
     size_t need = 0;  // the largest island a world's joints and bodies can make
     for (int w = 0; w < nw; ++w) {
       const int k = b->joint_off[w + 1] - b->joint_off[w];
-      if (k == 0) continue;
-      ++joint_worlds;
-      need = std::max(need, joint_lds_bytes(k, b->body_off[w + 1] - b->body_off[w]));
+      if (k > 0) need = std::max(need, joint_lds_bytes(k, b->body_off[w + 1] - b->body_off[w]));
     }
-    need = (need + 255) & ~(size_t)255;
-    if (need <= (size_t)kJointLdsMax && joint_worlds <= kCus * (kMaxLds / (int)need)) ctx->joint_lds = (int)need;
+    if (need <= (size_t)kJointLdsMax && nj <= kJointWaves * joint_lane_steps(b)) ctx->joint_lds = (int)align256(need);
   }
   if (!ctx->big.empty()) {  // scratch of the large-world path
     int *wb = nullptr, *bl = nullptr;
@@ -7630,6 +7663,8 @@ B2G_API int b2g_set_param(b2g_ctx* ctx, int32_t key, int32_t value) {
       return set_error(ctx, B2G_E_INVALID, "b2g_set_param: B2G_PARAM_SOLVE_WAVES_PER_CU is read-only");
     case B2G_PARAM_SEARCH_RUNS:
       return set_error(ctx, B2G_E_INVALID, "b2g_set_param: B2G_PARAM_SEARCH_RUNS is read-only");
+    case B2G_PARAM_JOINT_LDS:
+      return set_error(ctx, B2G_E_INVALID, "b2g_set_param: B2G_PARAM_JOINT_LDS is read-only");
     default: return set_error(ctx, B2G_E_INVALID, "b2g_set_param: unknown key " + std::to_string(key));
   }
   if (key == B2G_PARAM_COLLIDE_BLOCK && (value & (value - 1)) != 0)
@@ -7673,6 +7708,7 @@ B2G_API int b2g_get_param(b2g_ctx* ctx, int32_t key, int32_t* value) {
     case B2G_PARAM_COLLIDE_BLOCK: *value = ctx->collide_block; return B2G_OK;
     case B2G_PARAM_TREE_PAIRS: *value = ctx->tree_pairs; return B2G_OK;
     case B2G_PARAM_EVENTS: *value = ctx->ev_mask; return B2G_OK;
+    case B2G_PARAM_JOINT_LDS: *value = ctx->joint_lds; return B2G_OK;
     case B2G_PARAM_SEARCH_RUNS: *value = (int)ctx->isl_runs.size() | (int)ctx->pair_runs.size() << 8; return B2G_OK;
     case B2G_PARAM_SOLVE_WAVES_PER_CU: {
       // resident solver wavefronts per compute unit: 4 SIMDs x (512 VGPRs / VGPRs per lane), and
