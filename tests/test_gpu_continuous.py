@@ -152,3 +152,60 @@ def test_drop_in_world_listener_receives_the_sub_step_calls():
         sub_step_calls += int(np.count_nonzero(ei[:, L.EI_PHASE] == 3))
         log.clear()
     assert sub_step_calls > 0
+
+
+def peg_scene(pegs, shots):
+    """A board of static pegs (circles and boxes by turns) and, after them in fixture order, small bullets
+    and other fast bodies flying through it: sub-steps whose bodies meet proxies of any index."""
+    bodies = []
+    for k in range(pegs):
+        x, y = 1.1 * (k % 16) + (0.55 if k // 16 % 2 else 0.0), 1.0 * (k // 16)
+        shape = ("circle", 0.2) if k % 2 == 0 else ("box", 0.18, 0.18)
+        bodies.append({"type": "static", "position": (x, y), "angle": 0.2 * (k % 5), "linear_velocity": (0.0, 0.0),
+                       "angular_velocity": 0.0, "fixtures": [{"shape": shape, "density": 0.0, "friction": 0.2,
+                                                              "restitution": 0.6}]})
+    for k in range(shots):
+        shape = ("circle", 0.12) if k % 2 == 0 else ("box", 0.1, 0.12)
+        bodies.append({"type": "dynamic", "position": (-1.0 - 0.9 * (k // 8), 0.45 + 1.03 * (k % 8)), "angle": 0.3 * k,
+                       "linear_velocity": (70.0 + 5.0 * (k % 7), 12.0 - 3.0 * (k % 9)), "angular_velocity": 1.0 + k,
+                       "bullet": k % 3 == 0, "fixtures": [{"shape": shape, "density": 1.0, "friction": 0.2,
+                                                           "restitution": 0.7}]})
+    return {"gravity": (0.0, -10.0), "do_sleep": True, "warm_starting": True, "bodies": bodies}
+
+
+def _pairs(st):
+    return set(map(tuple, st.con_i[:, [L.CI_FA, L.CI_FB]].tolist()))
+
+
+@pytest.mark.parametrize("pegs,shots", [(104, 24), (105, 24), (168, 24)])
+def test_sub_steps_in_worlds_of_more_fixtures_than_lanes(pegs, shots):
+    """128, 129 and 192 fixtures: the sub-steps' passes over fixtures and contacts take several rounds of a
+    wavefront's lanes, the last one full or of one fixture, and their pair searches make contacts.  Each
+    step starts from the oracle's state (a body that grazes pegs at 90 m/s parts from any other
+    rounding of its run within a few steps)."""
+    batch = continuous_batch(peg_scene(pegs, shots))
+    assert batch.fix_d.shape[0] == pegs + shots
+    o = O.Oracle(batch)
+    e = N.Engine("fp64")
+    events = made = 0
+    for s in range(1, 25):
+        start = o.state()
+        e.upload(start)
+        e.stats(reset=True)
+        assert o.step(DT, 8, 3) == 0
+        e.step(DT, 8, 3)
+        st = e.stats(reset=True)
+        want = o.toi_stats(0)
+        assert (st["toi_calls"], st["toi_events"]) == want, (s, st["toi_calls"], st["toi_events"], want)
+        events += want[1]
+        ref, got = o.state(), e.download()
+        assert PU.same_contact_lists(got, ref), s
+        be = PU.body_errors(got, ref)
+        assert max(be[q] for q in PU.QUANTITIES) <= 1e-9, (s, be)
+        start.world_i[0, L.WI_FLAGS] &= ~L.WF_CONTINUOUS
+        p = O.Oracle(start)
+        p.step(DT, 8, 3)
+        made += len(_pairs(ref) - _pairs(p.state()))
+    print(pegs, shots, "toi events", events, "contacts made in sub-steps", made, flush=True)
+    assert events > 20 and made > 10
+    e.close()

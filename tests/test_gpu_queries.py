@@ -145,6 +145,28 @@ def test_queries_on_large_worlds_match_the_oracle(count):
     e.close()
 
 
+def test_ray_casts_over_worlds_on_both_sides_of_the_fixture_limit():
+    """Worlds of few fixtures, of 8192 (the last a wavefront takes) and of 8193 (a lane on the tree) in one
+    call, their rays interleaved."""
+    def grid(n):
+        boxes = [{"shape": ("polygon", [(x, y), (x + 0.6, y), (x + 0.5, y + 0.5)]), "density": 0.0, "friction": 0.2,
+                  "restitution": 0.0} for x, y in ((float(k % 128), float(k // 128)) for k in range(n))]
+        return {"gravity": (0.0, -10.0), "do_sleep": True, "warm_starting": True,
+                "bodies": [{"type": "static", "position": (-64.0, 0.0), "angle": 0.0, "linear_velocity": (0.0, 0.0),
+                            "angular_velocity": 0.0, "fixtures": boxes}]}
+    specs = [scenes.batch_world(3, 0, 20), grid(8193), scenes.batch_world(3, 1, 90), grid(8192), grid(65)]
+    state = builder.scenes_batch(specs)
+    assert np.diff(state.fix_off)[[1, 3]].tolist() == [8193, 8192]
+    e = engine_with(state)
+    rng = np.random.default_rng(12)
+    n = 203
+    worlds = (np.arange(n) % len(specs)).astype(np.int32)
+    segs = np.stack([rng.uniform(-60, 60, n), rng.uniform(0, 60, n), rng.uniform(-60, 60, n), rng.uniform(0, 60, n)], 1)
+    boxes = np.stack([segs[:, 0], segs[:, 1], segs[:, 0] + 2.0, segs[:, 1] + 2.0], 1)
+    check_against_oracle(state, e, worlds, boxes, segs)
+    e.close()
+
+
 def test_drop_in_world_queries_and_ray_cast_callbacks():
     import pypybox2d_amd as b2
     world = b2.World(gravity=(0, -10), do_sleep=True, continuous_physics=False)
