@@ -707,8 +707,6 @@ __global__ void __launch_bounds__(B) k_collide(Dev<T> d, int chunks) {
 // ---------------------------------------------------------------------------
 // per-world island search
 // ---------------------------------------------------------------------------
-// The 32-bit LDS address of a pointer into the workgroup's LDS (for LDS reads written in inline
-// assembly).
 // The lanes of one wavefront exchange body state through LDS between passes.
 // LDS instructions of a wavefront execute in issue order, so wavefront-scope
 // ordering (which emits no waits) is all a pass boundary needs.
@@ -800,11 +798,16 @@ __host__ __device__ inline size_t island_smem_bytes(int nb, int nf, int ccap) {
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;  // lev
   s += ((size_t)nb * 2 + 15) & ~(size_t)15;  // ibs
-  // free: a bit per contact slot, so that the same worlds fit whose joints the other path refuses
-  s += ((size_t)(ccap + 31) / 32 * 4 + 15) & ~(size_t)15;
   s += (size_t)kBlock * 4;
   s += 64 * 4;  // misc: 16 scalars, 32 class counts, spare
   return s;
+}
+
+// The worlds whose search is by LDS are those that leave a bit per contact slot of it free: a world with
+// joints that does not fit is refused, so the limit is part of what a caller sees and does not move with
+// what the search happens to hold.
+inline bool island_search_fits(int nb, int nf, int ccap) {
+  return island_smem_bytes(nb, nf, ccap) + (((size_t)(ccap + 31) / 32 * 4 + 15) & ~(size_t)15) <= (size_t)kMaxLds;
 }
 
 // Exclusive scan of a[0..n) in place by one workgroup; returns the total.  scratch: a value per wavefront.
@@ -1264,7 +1267,7 @@ __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_i
   // contacts before them.  A lane polls its contacts in list order, which every dependency follows;
   // cur holds a body's contacts done << 16 | the last one's level.
   for (int i = tid; i < nb; i += kBlock) L.cur[i] = 0;
-  for (int c = tid; c < nci_tot; c += kBlock) {  // (the lane's own records: no barrier between)
+  for (int c = tid; c < nci_tot; c += kBlock) {  // (written per body by any lane, before the barrier above)
     const uint2 r = d.i_rank[cb + c];
     L.adj[2 * c] = r.x | d.i_order[cb + c] << 16;
     L.adj[2 * c + 1] = r.y;
@@ -2873,6 +2876,8 @@ __global__ void __launch_bounds__(kSolveBlock) __attribute__((amdgpu_waves_per_e
 // 0.38 -> 0.16 ms.  With 128 VGPRs, four wavefronts per SIMD, the record spills and the FP32 pass
 // takes 0.70 us.
 // ---------------------------------------------------------------------------
+// The 32-bit LDS address of a pointer into the workgroup's LDS (for LDS reads written in inline
+// assembly).
 template <typename P>
 __device__ __forceinline__ uint32_t lds_addr(P* p) {
   return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) P*)p);
@@ -5035,7 +5040,7 @@ __device__ inline void toi_init_velocity(ToiScratch& S, int k) {
 
 // What lane 0 tells the other lanes.
 struct ToiVars {
-  int st, nbi, nci, nmove, full, used;
+  int st, nbi, nci, full;
 };
 struct ToiLds {
   ToiScratch S;
@@ -6284,7 +6289,8 @@ static int upload_batch(b2g_ctx* ctx, const b2g_batch* b) {
   for (int w = 0; w < nw; ++w) {
     const int wnb = ctx->body_off[w + 1] - ctx->body_off[w], wnf = ctx->fix_off[w + 1] - ctx->fix_off[w];
     const size_t si = island_smem_bytes(wnb, wnf, ctx->con_cap[w]), sp = pairs_smem_bytes(wnf, ctx->con_cap[w]);
-    if (ctx->large_worlds || ctx->con_cap[w] >= 65535 || si > (size_t)kMaxLds || sp > (size_t)kMaxLds) {
+    if (ctx->large_worlds || ctx->con_cap[w] >= 65535 || !island_search_fits(wnb, wnf, ctx->con_cap[w]) ||
+        sp > (size_t)kMaxLds) {
       w_big[w] = 1;
       ctx->big.push_back(w);
       ctx->smem_big = std::max(ctx->smem_big, (size_t)((wnb + 1) / 2) * 4);  // 16-bit union-find parents
