@@ -7548,6 +7548,7 @@ B2G_API int b2g_step(b2g_ctx* ctx, double dt, int vel_iters, int pos_iters) {
 B2G_API int b2g_step_n(b2g_ctx* ctx, int n, double dt, int vel_iters, int pos_iters, int use_graph) {
   if (!ctx || !ctx->dev) return set_error(ctx, B2G_E_INVALID, "no batch uploaded");
   ctx->status_ok = false;
+  ctx->tree_dirty = true;  // (also where a captured step is launched again)
   if (ctx->split) return set_error(ctx, B2G_E_INVALID, "a step begun by b2g_step_collide is not finished");
   if (n < 0 || vel_iters < 0 || pos_iters < 0) return set_error(ctx, B2G_E_INVALID, "negative count");
   hipSetDevice(ctx->device);

@@ -129,6 +129,26 @@ def test_batched_queries_over_many_worlds_match_the_oracle():
     e.close()
 
 
+@pytest.mark.parametrize("count", [1, 150])
+def test_queries_after_replayed_steps_see_the_moved_bodies(count):
+    """Queries and ray casts before and after more launches of a captured step: worlds of 56 fixtures, and of
+    8400, whose rays walk the tree too."""
+    batch = builder.scene_batch(scenes.pyramids(count))
+    dyn = batch.body_i[:, L.BI_TYPE] == L.DYNAMIC
+    batch.body_d[dyn, L.BD_V_X] += 60.0
+    e = engine_with(batch)
+    rng = np.random.default_rng(8)
+    total = 0
+    for part in range(3):
+        e.step_n(20, DT, 8, 3, graph=True)
+        state = e.download()
+        hits = check_against_oracle(state, e, *random_queries(rng, state, 100))
+        print(count, part, "query results and ray hits", hits, flush=True)
+        total += hits[0]
+    assert total > 50
+    e.close()
+
+
 @pytest.mark.parametrize("count", [200, 640])
 def test_queries_on_large_worlds_match_the_oracle(count):
     """One world of 200 pyramids (11 200 proxies: the LDS sort) and of 640 (36 480 proxies: the
