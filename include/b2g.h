@@ -88,7 +88,12 @@ B2G_API int b2g_counts(b2g_ctx* ctx, int32_t* counts);
 
 /* Copy the full state back (bodies, fat AABBs, ordered contacts with their
    manifolds and impulses, move buffer, joint records) into caller arrays.
-   Replaces reading Body/Contact/Manifold/Joint attributes after World.step. */
+   Replaces reading Body/Contact/Manifold/Joint attributes after World.step.
+   The records pass through pinned host memory that the context keeps until
+   b2g_destroy: a quarter more than the largest state read, at most 80 MB and the
+   worlds' scalars.  The first download of an uploaded batch also allocates 16 bytes
+   per body and 4 per contact slot on the device.  b2g_ray_cast (closest hits) uses the
+   same pinned memory, 105 bytes per ray and at most 27 MB. */
 B2G_API int b2g_download(b2g_ctx* ctx, b2g_batch_out* out);
 
 /* memcpy of host arrays by up to 8 threads (from 4 MB on), for the copies of a
@@ -171,7 +176,9 @@ B2G_API int b2g_last_error(b2g_ctx* ctx, char* buf, size_t n);
                           wavefronts (64 lanes in b2g_island_times), while their
                           load, in workgroups of 512 lanes weighted by island size,
                           is at most this (0..2^20, default 768; 0: never, and
-                          never with a heavy class above 9).  Results do not
+                          never with a heavy class above 9 or more than 4103
+                          velocity iterations).  Islands of 3 to 30 contacts take a
+                          wavefront only while those are few.  Results do not
                           depend on it. */
 #define B2G_PARAM_GROUP_LOAD 15
 /* B2G_PARAM_JOINT_LDS    (read only) bytes of LDS in which a wavefront each solves the

@@ -4733,8 +4733,9 @@ __global__ void __launch_bounds__(256) k_query_aabb(Dev<T> d, int nq, const int*
 // casts the ray at 64 of their shapes at a time.  Worlds of more than kRayWaveFixtures fixtures
 // (2 KB of boxes a step of 64, from L2) walk the tree instead, a lane per ray: a lane's walk is a
 // chain of dependent reads with a stack in scratch, 1088 us for 32 rays in each of 512 worlds of 32
-// to 512 bodies, where the whole call takes 124 us now (1352 before).  One world, 16384 rays: 178 us at 3360 fixtures
-// and growing in proportion, against 554 to 573 us by the tree at 4200 to 11200; 1000 rays 42 against 457 us.
+// to 512 bodies, where the whole call takes 122 us now (1330 before).  One world, us a call by wavefronts / by the tree
+// with device staging: 3360 fixtures 42 / 539 for 1000 rays, 175 / 645 for 16384, 2545 / 5375 for 262144; 7840 fixtures
+// 62 / 589, 258 / 672, 3597 / 5680.
 constexpr int kRayWaveFixtures = 8192;
 constexpr int kRayWaves = 4;  // rays per workgroup
 
@@ -4877,7 +4878,9 @@ __global__ void __launch_bounds__(256) k_ray_cast(Dev<T> d, int nr, const int* r
 // fixtures, the island's records; lane 0 keeps what is ordered.  The island and the shapes'
 // vertices are in LDS.  Bound by the longest time_of_impact of a round and by the ordered parts'
 // latency.  All of it on one lane, with the island in HBM, took 3.0 ms a step for 31 worlds of 20
-// fast bodies and 0.2 to 0.6 ms for the settled 10-row pyramid; this takes 1.4 and 0.02 ms.
+// fast bodies and 0.2 to 0.6 ms for the settled 10-row pyramid; this takes 1.3 and 0.08 ms (0.27 at most).
+// The 37 KB of LDS let four worlds run on a compute unit; 4096 worlds of fast bodies take 8.7 ms a step, on one
+// lane each 23.9, 4096 piles 1.4 and 2.4 (31 worlds: 1.9 and 4.3).
 // ---------------------------------------------------------------------------
 constexpr int kToiContacts = 32;     // settings.py:79 (MAX_TOI_CONTACTS)
 constexpr int kToiBodies = 64;       // 2 * MAX_TOI_CONTACTS
