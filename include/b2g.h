@@ -197,8 +197,8 @@ B2G_API int b2g_profile_step(b2g_ctx* ctx, int n, double dt, int vel_iters, int 
 /* With B2G_PARAM_ISLAND_TIMES on: the islands the last step solved, in the
    solver's queue order, as 6 int64 each: start and end (ns, device wall
    clock), contacts | bodies << 32, lanes | period << 32 (the lanes that
-   solved it: a team's size, 1 for one lane per island, 0 for a team island
-   whose state did not fit the team's LDS share or that has joints; and its
+   solved it: a team's size, 64 also for a group of wavefronts, 1 for one lane
+   per island, 0 for a team island whose state did not fit the team's LDS share or that has joints; and its
    sweep period, the lag in dependency levels between consecutive sweeps,
    which with the iteration counts predicts the island's passes), the end of
    its velocity iterations (ns) and the number of position iterations it ran

@@ -1,8 +1,8 @@
 // b2g_engine.hip -- batched MI355X (gfx950) contact pipeline and its C-ABI.
 //
 // One call of b2g_step advances every world of a batch by one
-// World.step(dt, velocity_iterations, position_iterations) (world.py:307-354)
-// with continuous physics off.  Per step the device runs:
+// World.step(dt, velocity_iterations, position_iterations) (world.py:307-354).
+// Per step the device runs (and k_toi at the end, where continuous physics is on):
 //
 //   k_collide   one lane per contact slot: ContactManager.collide
 //               (contact_manager.py:174-223) for contacts with an awake
@@ -12,8 +12,10 @@
 //               awake gating (only worlds holding sleeping bodies), then the
 //               island search of World._solve (world.py:494-580) over an
 //               LDS-resident contact graph, in the reference's DFS order.
-//   k_solve     one lane per island, pulled from a device queue: Island.solve
-//               (island.py:65-179) with ContactSolver (contact.py:375-864).
+//   k_solve, k_solve_group, k_solve_joints*
+//               islands from a device queue, by a lane, a team of lanes or whole
+//               wavefronts each: Island.solve (island.py:65-179) with
+//               ContactSolver (contact.py:375-864) and the joints.
 //   k_sync      one lane per fixture: Body._synchronize_fixtures + move_proxy
 //               (body.py:898-904, fixture.py:287-298, dynamictree.py:152-188)
 //               with FP64 swept AABBs.
@@ -842,8 +844,8 @@ __device__ int block_exclusive_scan(int* a, int n, int* scratch) {
 }
 
 // B threads per workgroup: 256, or 128 for worlds whose LDS footprint lets more than five
-// workgroups share a CU (the one-lane walk dominates the kernel, so more worlds in flight
-// per CU outweigh the slower wide phases).
+// workgroups share a CU (the walk, one wavefront's, dominates the kernel, so more worlds in
+// flight per CU outweigh the slower wide phases).
 template <typename T, int B>
 __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(5))) k_islands(Dev<T> d, int w_first) {
   constexpr int kBlock = B;
